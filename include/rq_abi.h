@@ -263,8 +263,9 @@ int rq_fused_decode_noalloc(const void *q, int32_t dtype, int64_t num_seqs, int3
                             void *stream);
 
 /*
- * Causal prefill attention over the packed cache on int8 MFMA (Q K^T and P V),
- * for any number of sequences in one launch.  Query token i of sequence b sits
+ * Causal prefill attention over the packed cache on 16-bit MFMA, for any number
+ * of sequences in one launch (the reference's product runs on int8 operands; here
+ * the rotated queries and the dequantized K are multiplied exactly in the q dtype).  Query token i of sequence b sits
  * at position seq_lens[b] - q_len_b + i, where q_len_b = cu_seqlens_q[b+1] -
  * cu_seqlens_q[b]; it attends to cache positions <= its own.
  *
@@ -277,7 +278,7 @@ int rq_fused_decode_noalloc(const void *q, int32_t dtype, int64_t num_seqs, int3
  * (q rows and the rotation 16-byte aligned).  max_q_len bounds every q_len_b; max_seq_len bounds every seq_lens[b] (keys
  * past it are not read).  workspace: rq_int8_prefill_workspace_bytes() bytes,
  * 16-byte aligned, no initialisation needed (two launches: a pack kernel
- * decodes the cache's K/V into int8 tile images there, the attention kernel
+ * decodes the cache's K/V into tile images there, the attention kernel
  * streams them).  Other arguments as for rq_fused_decode.
  */
 int rq_int8_prefill(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,
@@ -295,7 +296,7 @@ int rq_int8_prefill(const void *q, int32_t dtype, int64_t total_q, int32_t num_q
                     void *workspace, int64_t workspace_bytes,
                     void *stream);
 
-/* Workspace bytes rq_int8_prefill needs: one int8 tile image (33 KB)
+/* Workspace bytes rq_int8_prefill needs: one tile image (33 KB)
  * per 64 keys of max_seq_len, per sequence and kv head.  No counterpart in the
  * reference, which decodes K/V inside its attention kernel. */
 int64_t rq_int8_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads, int64_t max_seq_len);

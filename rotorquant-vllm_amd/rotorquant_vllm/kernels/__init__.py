@@ -280,7 +280,7 @@ _ws_retired: list = []
 
 def shared_workspace(device, kind: str, nbytes: int) -> torch.Tensor:
     """Device scratch of one kind per device ("decode": split-KV partials, query
-    operands, tile descriptors; "prefill": int8 tile images), shared by every call
+    operands, tile descriptors; "prefill": tile images), shared by every call
     on the device's stream (calls run one after another; every call rewrites what
     it reads).  When a call needs more, a larger buffer replaces it and the old one
     is kept allocated until the process ends, so a HIP graph that captured its
@@ -391,7 +391,7 @@ def fused_paged_rq_decode_launcher(q: torch.Tensor, kv_cache: torch.Tensor, bloc
 
 
 # ---------------------------------------------------------------------------
-# INT8 prefill
+# Fused prefill
 # ---------------------------------------------------------------------------
 
 def _single_cu_seqlens(device, num_tokens: int) -> torch.Tensor:
@@ -408,15 +408,17 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
                                 cu_seqlens_q: torch.Tensor | None = None,
                                 max_q_len: int | None = None, max_seq_len: int | None = None,
                                 workspace: torch.Tensor | None = None, dense3: bool = False) -> torch.Tensor:
-    """Causal prefill attention from the packed cache with Q K^T and P V on int8 MFMA.
+    """Causal prefill attention from the packed cache.
 
-    Reference: src/rotorquant_vllm/triton/fused_paged_rq_int8_prefill.py:247-363.
+    Reference: src/rotorquant_vllm/triton/fused_paged_rq_int8_prefill.py:247-363 (its
+    products run on int8 operands; here K and the rotated query are multiplied exactly in
+    q's dtype, which is more precise and on gfx950 faster: rq_prefill.hip).
     q: (num_tokens, H_Q, D); block_table (num_seqs, max_blocks) int32; seq_lens
     (num_seqs,) int32 total context lengths (new tokens included).
     cu_seqlens_q (num_seqs + 1,) int32 splits q among sequences; without it
     there must be one sequence (as in the reference).
     max_seq_len bounds every seq_lens entry (default: the block table's capacity)
-    and sizes the int8 tile-image workspace; workspace may be passed to reuse a
+    and sizes the tile-image workspace; workspace may be passed to reuse a
     buffer of rq_int8_prefill_workspace_bytes bytes.  dense3: the cache holds the
     dense 3-bit index layout.
     """

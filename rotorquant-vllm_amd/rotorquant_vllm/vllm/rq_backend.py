@@ -13,7 +13,7 @@ librq_hip.so (include/rq_abi.h):
 
     compress + store  -> rq_compress_store   (one fused K+V launch, writes slots)
     decode            -> rq_fused_decode     (Q and output rotation inside)
-    prefill           -> rq_int8_prefill     (int8 MFMA, multi-sequence)
+    prefill           -> rq_int8_prefill     (tile images + MFMA, multi-sequence)
     non-fused path    -> rq_paged_attention  (K/V dequantized to the q dtype in
                          LDS, 16-bit MFMA; head_size 128; decodes), and for
                          longer queries rq_paged_prefill (the same arithmetic,
