@@ -21,19 +21,22 @@
 // aligned mask with seqused_k); otherwise all seq_lens[b] keys.
 //
 // One workgroup per (query block, kv head, sequence); its waves are (query
-// head of the GQA group, 16-position group), as in rq_prefill.hip.  The
+// head of the GQA group, position group).  WIDE (some query is longer than 16 tokens):
+// groups of 32 positions and rq_prefill.hip's tile steps (rq_attn_tile.h), so that both kernels
+// give the same bits; else groups of 16.  The
 // workgroup decodes each 64-key tile of its (sequence, kv head) from the
 // packed slots into a double-buffered LDS tile (K rows in the q dtype, fp16
 // V'^T rows): while tile t is computed, tile t+1's packed bytes are copied
 // cache -> LDS staging with direct global -> LDS copies, and decoded into the
 // other buffer after it.  No workspace, no decompressed copy of the cache.
 //
-// MFMA v_mfma_f32_16x16x32_{bf16,f16} for S^T = K Q^T (wave64, lane l,
+// Groups of 16: MFMA v_mfma_f32_16x16x32_{bf16,f16} for S^T = K Q^T (wave64, lane l,
 // g = l / 16, col = l % 16), four k-steps of 32 head dims:
 //   A (16 keys x 32 dims): lane holds key 16b + col, dims 32s + 8g .. +7;
 //   B (32 dims x 16 positions): lane holds position col, the same dims;
 //   C: lane (g, col) holds position col's scores of keys 16b + 4g + i.
 #include <algorithm>
+#include <type_traits>
 
 #include "rq_attn_tile.h"
 
@@ -44,12 +47,13 @@ namespace {
 constexpr int kD = kAttnD;
 constexpr int kKT = kAttnKT;
 constexpr int kPQ = kAttnPQ;
+constexpr int kPW = kAttnPW;
 
 // LDS, per workgroup:
 //   two tile buffers: K rows (64 keys x 256 bytes in the q dtype, 16-byte piece
 //     c = dims 8c .. 8c+7 of key r, in the order e0 e2 e4 e6 e1 e3 e5 e7, at
 //     r * 256 + 16 * (c ^ (r & 15)): the 16 keys one MFMA operand read touches
-//     hit 16 distinct piece slots), then V'^T (vt_piece);
+//     hit 16 distinct piece slots; the same as kw_piece), then V'^T (vt_piece or vw_piece);
 //   staging: the next tile's packed bytes as copied from the cache -- K index
 //     dwords [key][16], V index dwords [key][16], K norms [key], V norms [key];
 //   slot offsets of the keys of the tile staged next.
@@ -90,15 +94,17 @@ struct AttnArgs {
     int rot_block;
     int causal;
     float score_scale;  // sm_scale * log2(e)
-    int qb;             // query positions per workgroup (= 16 * position groups)
+    int qb;             // query positions per workgroup (= 16 or 32 * position groups)
     int npg;            // position groups per workgroup
     int ncomp;          // waves that compute (query head, position group); the rest only decode tiles
     void *out;
     int64_t o_st, o_sh;
 };
 
-template <int DT>
-__global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) {
+// (WIDE keeps 2 waves per SIMD, as the prefill's kernel; the narrow form fits 4.)
+template <int DT, bool WIDE>
+__global__ __launch_bounds__(64 * kMaxWaves) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 4))) void paged_attn_kernel(AttnArgs a) {
+    constexpr int kP = WIDE ? kPW : kPQ;  // positions per wave
     int qblk, hy;
     int64_t seq;
     attn_work_item(qblk, hy, seq);
@@ -114,16 +120,17 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int nwaves = nthr >> 6;
-    const int g = lane >> 4, col = lane & 15;
+    const int g = lane >> (WIDE ? 5 : 4), col = lane & (kP - 1);
     const int gw = a.G / a.hsplit;                   // query heads of this workgroup
     const int gh = hpart * gw + wave / a.npg;        // query head inside the GQA group
-    const int pg = wave % a.npg;                     // 16-position group
+    const int pg = wave % a.npg;                     // position group
     const int hq = h * a.G + gh;
-    const int i0 = qblk * a.qb + pg * kPQ;  // first query index of this wave
+    const int i0 = qblk * a.qb + pg * kP;  // first query index of this wave
     const bool wave_active = wave < a.ncomp && i0 < T;
     const int my_pos = pos_base + i0 + col;
-    // V'^T pieces of this lane (dim col, pieces g and 4 + g)
-    const int voff0 = vt_piece(col, g), voff1 = vt_piece(col, 4 + g);
+    // V'^T pieces of this lane (narrow: dim col, pieces g and 4 + g)
+    [[maybe_unused]] const int voff0 = vt_piece(col, g), voff1 = vt_piece(col, 4 + g);
+    [[maybe_unused]] const WideOffsets wo(g, col);
 
     // Keys [0, kv_end) may be visible to some query of the workgroup.
     const int last_i = min(T, (qblk + 1) * a.qb) - 1;
@@ -132,6 +139,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
 
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ float ktab[16], vtab[16];
+    __shared__ float4 rot[kAttnD];
+    load_rotation(rot, a.R, tid);
     if (tid < 16) {
         ktab[tid] = tid < a.nkc ? a.kc[tid] : 0.f;
         vtab[tid] = tid < a.nvc ? a.vc[tid] : 0.f;
@@ -238,7 +247,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
                 const int tq = u & 15, dw = u >> 4;
                 const int t0 = 4 * tq;
                 const int b = t0 >> 4, gg = (t0 >> 2) & 3;
-                const int piece = 4 * (b >> 1) + gg, elem_off = 8 * (b & 1);
+                const int piece = WIDE ? vw_quad_piece(tq) : 4 * (b >> 1) + gg;
+                const int elem_off = WIDE ? vw_quad_byte(tq) : 8 * (b & 1);
                 uint32_t x[4];
                 float nrm[4];
 #pragma unroll
@@ -259,7 +269,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
                             const float v = Elem<DT>::to_f32(Elem<DT>::from_f32(opaque(vtab[idx] * nrm[i])));
                             e[i] = f32_to_f16_bits(v * vs);
                         }
-                        *reinterpret_cast<uint2 *>(tb + kTVt + vt_piece(d, piece) + elem_off) =
+                        *reinterpret_cast<uint2 *>(tb + kTVt + (WIDE ? vw_piece(d, piece) : vt_piece(d, piece)) + elem_off) =
                             make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
                     }
                 }
@@ -277,29 +287,20 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
     if (n_tiles > 0) stage();
     if (n_tiles > 1) issue_bt(1);
 
-    // ---- Q^T operand: position i0 + col, k-step s = dims 32s + 8g .. +7 of q_rot ----
-    u32x4 qop[4];
-    {
-        const int qi = i0 + col;
-        const bool qvalid = wave_active && qi < T;
-        const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (qvalid ? qi : 0)) * a.q_st +
-                               (int64_t)hq * a.q_sh;
+    // ---- Q^T operand: position i0 + col (narrow: k-step s = dims 32s + 8g .. +7 of q_rot) ----
+    u32x4 qop[WIDE ? 8 : 4];
+    const bool qvalid = wave_active && i0 + col < T;
+    const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (qvalid ? i0 + col : 0)) * a.q_st +
+                           (int64_t)hq * a.q_sh;
+    if constexpr (WIDE) {
+        wide_query_load(qop, qrow, qvalid, g);
+        wide_query<DT, true>(qop, rot, a.rot_block, g);
+    } else {
 #pragma unroll
         for (int s_ = 0; s_ < 4; ++s_) {
             const int base = 32 * s_ + 8 * g;
-            const uint4 rw = qvalid ? *reinterpret_cast<const uint4 *>(qrow + base) : make_uint4(0, 0, 0, 0);
-            const uint32_t w16[4] = {rw.x, rw.y, rw.z, rw.w};
-            float xin[8], qr[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) xin[k] = Elem<DT>::to_f32((w16[k >> 1] >> (16 * (k & 1))) & 0xffffu);
-            rotate_q8<DT>(xin, base, a.R, a.rot_block, qr);
-            // dims in the K rows' order e0 e2 e4 e6 e1 e3 e5 e7
-            uint32_t pk[4];
-            constexpr int ord[8] = {0, 2, 4, 6, 1, 3, 5, 7};
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                pk[k] = Elem<DT>::from_f32(qr[ord[2 * k]]) | (Elem<DT>::from_f32(qr[ord[2 * k + 1]]) << 16);
-            qop[s_] = u32x4{pk[0], pk[1], pk[2], pk[3]};
+            const u32x4 raw = qvalid ? *reinterpret_cast<const u32x4 *>(qrow + base) : u32x4{0u, 0u, 0u, 0u};
+            qop[s_] = a.rot_block == 4 ? rotate_q8<DT, 4, true>(raw, base, rot) : rotate_q8<DT, 2, true>(raw, base, rot);
         }
     }
 
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
         __syncthreads();  // tile 0 decoded, offsets of tile 1
     }
 
-    AttnState st;
+    std::conditional_t<WIDE, WideState, AttnState> st;
     st.init();
     for (int ti = 0; ti < n_tiles; ++ti) {
         const int k0 = ti * kKT;
@@ -322,7 +323,29 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
         if (ti + 2 < n_tiles) issue_bt(ti + 2);  // its block-table entries, read after the compute
         const uint8_t *tb = lds + (ti & 1) * kTileBytes;
         // (every wave reaches the barriers below)
-        if (wave_active && (!a.causal || k0 <= pos_base + i0 + kPQ - 1)) {
+        if (wave_active && (!a.causal || k0 <= pos_base + i0 + kP - 1)) {
+            // causal and tile-end mask: key < min(k0 + nk, position + 1)
+            const bool full = nk == kKT && (!a.causal || k0 + kKT - 1 <= pos_base + i0);
+            const int lim = (a.causal ? min(k0 + nk, my_pos + 1) : k0 + nk) - (k0 + 4 * g);
+            if constexpr (WIDE) {
+                f32x16 s[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) s[b] = mfma32<DT>(wide_k(tb + kTK, wo, ks, b), qop[ks], s[b]);
+                if (!full) wide_mask(s, lim);
+                const float bias = wide_max(st, wide_lane_max(s), a.score_scale, e_cur);
+                uint32_t pop[16];
+                float l = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) wide_exp_pair(s, i, a.score_scale, bias, pop, l);
+                wide_add_sum(st, l, e_cur);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m)
+                        st.acc[m] = mfma32<RQ_DTYPE_F16>(wide_v(tb + kTVt, wo, t, m), wide_p(pop, t), st.acc[m]);
+            } else {
             // ---- S^T = K Q^T for 4 key blocks of 16 ----
             float s[16];
 #pragma unroll
@@ -337,14 +360,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) s[4 * b + i] = c[i];
             }
-            // causal and tile-end mask: key < min(k0 + nk, position + 1)
-            const bool full = nk == kKT && (!a.causal || k0 + kKT - 1 <= pos_base + i0);
             if (!full) {
-                const int lim = (a.causal ? min(k0 + nk, my_pos + 1) : k0 + nk) - (k0 + 4 * g);
 #pragma unroll
                 for (int j = 0; j < 16; ++j) s[j] = (16 * (j >> 2) + (j & 3)) < lim ? s[j] : -INFINITY;
             }
             softmax_pv(st, s, a.score_scale, 1.f, e_cur, tb + kTVt, voff0, voff1, rowsum_operand(e_cur, col));
+            }
         }
         if (more) {
             wait_copies<0>();
@@ -356,10 +377,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void paged_attn_kernel(AttnArgs a) 
     }
     if (!wave_active) return;
 
-    const float inv_l = attn_inv_l(st);
-    if (i0 + col >= T) return;
-    uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + i0 + col) * a.o_st + (int64_t)hq * a.o_sh;
-    store_rotated<DT>(st, inv_l, orow, a.R, a.rot_block, g);
+    const bool ovalid = i0 + col < T;
+    uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + (ovalid ? i0 + col : 0)) * a.o_st + (int64_t)hq * a.o_sh;
+    if constexpr (WIDE) {
+        wide_store<DT>(st, ovalid, orow, rot, a.rot_block, g);
+    } else {
+        const float inv_l = attn_inv_l(st);
+        if (!ovalid) return;
+        if (a.rot_block == 4) store_rotated<DT, 4>(st, inv_l, orow, rot, g);
+        else store_rotated<DT, 2>(st, inv_l, orow, rot, g);
+    }
 }
 
 }  // namespace
@@ -426,30 +453,32 @@ extern "C" int rq_paged_attention(const void *q, int32_t dtype, int64_t total_q,
     a.causal = causal != 0;
     a.score_scale = sm_scale * kAttnLog2e;
     // GQA groups of more than kMaxWaves heads go to hsplit workgroups per kv head
-    // (the smallest split into equal parts of at most kMaxWaves heads); then
-    // 16-position groups per workgroup: up to kMaxWaves waves for long queries,
-    // at least kMinWaves waves (they share the tile decode).  When every query is
-    // short (one position group), the workgroup has kMaxWaves waves anyway: the
-    // waves past the GQA group's only decode tiles, which is most of a
-    // decode-shaped call's time.
+    // (the smallest split into equal parts of at most kMaxWaves heads).  When every query is
+    // short (one 16-position group), the workgroup has kMaxWaves waves anyway: the waves past
+    // the GQA group's only decode tiles, which is most of a decode-shaped call's time.
+    // Longer queries take groups of 32 positions, as many as make kMinWaves waves (they share
+    // the tile decode).
     a.hsplit = 1;
     while (a.G % a.hsplit != 0 || a.G / a.hsplit > kMaxWaves) ++a.hsplit;
     const int gw = a.G / a.hsplit;
-    a.npg = max_q_len > kPQ ? std::max(1, kMaxWaves / gw) : 1;
-    if (max_q_len > kPQ)
-        while (gw * a.npg < kMinWaves) ++a.npg;
-    a.qb = kPQ * a.npg;
+    const bool wide = max_q_len > kPQ;
+    a.npg = wide ? (kMinWaves + gw - 1) / gw : 1;
+    a.qb = (wide ? kPW : kPQ) * a.npg;
     a.ncomp = gw * a.npg;
     a.out = out;
     a.o_st = out_stride_tok;
     a.o_sh = out_stride_head;
-    const int nwaves = max_q_len > kPQ ? a.ncomp : kMaxWaves;
+    const int nwaves = wide ? a.ncomp : kMaxWaves;
     dim3 grid((unsigned)((max_q_len + a.qb - 1) / a.qb), (unsigned)(a.H * a.hsplit), (unsigned)num_seqs);
     const size_t lds = kLdsBytes;
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == RQ_DTYPE_BF16)
-        hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_BF16>), grid, dim3(64 * nwaves), lds, st, a);
-    else
-        hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_F16>), grid, dim3(64 * nwaves), lds, st, a);
+    const dim3 block(64 * nwaves);
+    if (dtype == RQ_DTYPE_BF16) {
+        if (wide) hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_BF16, true>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_BF16, false>), grid, block, lds, st, a);
+    } else {
+        if (wide) hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_F16, true>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((paged_attn_kernel<RQ_DTYPE_F16, false>), grid, block, lds, st, a);
+    }
     return check_launch("paged_attn_kernel");
 }

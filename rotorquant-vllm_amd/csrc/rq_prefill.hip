@@ -25,30 +25,22 @@
 //   with 11-bit operands on both sides: V' = V * 2^-e_tile in fp16, V the
 //   reference's centroid * norm rounded to the q dtype (:224), 2^e_tile above the
 //   64-key tile's largest v norm, and P' = p * 2^(e_tile - e_run) in fp16, e_run
-//   the largest e_tile so far (acc is rescaled when it grows); the row sum is a
-//   17th MFMA row of 2^-e_tile.
+//   the largest e_tile so far (acc is rescaled when it grows); the row sum is taken in
+//   fp32 before P' is rounded.
 //
 // Two kernels per call:
 //   * prefill_pack_kernel decodes every 64-key tile of every (sequence, kv head)
 //     once into a "tile image" in the caller's workspace: K rows in the q dtype,
 //     fp16 V'^T rows, the tile's V exponent, laid out exactly as the attention
 //     kernel keeps them in LDS;
-//   * prefill_attn_kernel: one workgroup per (query block of QB positions, kv
-//     head, sequence); its waves are (query head of the GQA group, 16-position
-//     group).  It streams the tile images of its sequence and kv head into a
-//     double-buffered LDS area with direct global -> LDS copies (the copy of
-//     tile t+1 runs while tile t is computed), so the inner loop is MFMA and
-//     softmax only.
-// MFMA v_mfma_f32_16x16x32_{bf16,f16} (wave64, lane l, g = l / 16):
-//   A (16 x 32): lane holds row l % 16, k = 8g .. 8g+7 (16 bytes)
-//   B (32 x 16): lane holds col l % 16, k = 8g .. 8g+7
-//   C (16 x 16): lane holds col l % 16, rows 4g .. 4g+3
-// S^T = K Q^T: rows = 16 keys of a key block, cols = 16 query positions; lane
-// (g, col) then holds the scores of keys 16b + 4g + i (b, i = 0..3).
-// O^T = V^T P^T, two k-steps per tile: k-step s, element j of lane
-// group g is key 32s + 4g + j (j < 4) or 32s + 16 + 4g + j - 4 (j >= 4) --
-// exactly the scores the lane holds, so P needs no transpose.
+//   * prefill_attn_kernel: a wave takes 32 query positions of one head, a workgroup
+//     four consecutive (position group, query head) units of a (sequence, kv head).
+//     It streams the tile images of its sequence and kv head into a double-buffered
+//     LDS area with direct global -> LDS copies (the copy of tile t+1 runs while tile
+//     t is computed), so the inner loop is MFMA and softmax only (wide_tile in
+//     rq_attn_tile.h, with the MFMA layouts).
 #include <algorithm>
+#include <type_traits>
 
 #include "rq_attn_tile.h"
 
@@ -56,7 +48,8 @@ namespace rq {
 
 constexpr int kPD = kAttnD;   // head_dim
 constexpr int kKT = kAttnKT;  // keys per tile
-constexpr int kPQ = kAttnPQ;  // query positions per wave
+constexpr int kPW = kAttnPW;  // query positions per wave
+constexpr int kWaves = 4;     // waves of an attention workgroup
 constexpr float kLog2eP = kAttnLog2e;
 
 struct PrefillArgs {
@@ -78,33 +71,20 @@ struct PrefillArgs {
     int rot_block;
     float score_scale;  // sm_scale * log2(e)
     int causal;         // 0: every query sees all seq_lens[b] keys
-    int qb;             // query positions per workgroup (= 16 * position groups)
-    int npg;            // position groups per workgroup
-    int flat;           // 1: workgroups of 8 waves over the sequence's (position group, query head) units
     int64_t max_tiles;  // tile images per (sequence, kv head) in the workspace
     uint8_t *ws;        // tile images [num_seqs][H][max_tiles][kImBytes]
     void *out;
     int64_t o_st, o_sh;
 };
 
-// Tile image (bytes), the same in the workspace and in LDS.  Rows are unpadded;
-// their 16-byte pieces are stored XOR-swizzled so that the ds_read_b128 operand
-// reads of an MFMA (16 lanes: 16 rows, one piece each) run without bank
-// conflicts.  Padded pitches of 144 / 80 bytes measured two-way conflicts on
-// gfx950; these swizzles measured conflict-free (same speed as contiguous reads).
-//   K row r, piece c (0..7):   r * 128 + 16 * (c ^ (r & 7))
-//   V^T row d, piece c (0..7): the same (8 keys of 16 bits per piece)
-// K rows: dtype(centroid * norm) as two [64 keys][64 dims] halves of 16-bit values (piece
-// c of key r's half h holds dims 64h + 8c .. +7 in order).
-constexpr int kKP = kPD;                            // row pitch
-constexpr int kImK = 0;                             // [2][64 keys][64 dims] q dtype
-constexpr int kImVt = kImK + 2 * kKT * kKP;         // [128 dims][64 keys] fp16 V', keys in MFMA k order
-__host__ __device__ constexpr int k_piece(int r, int c) { return r * kKP + 16 * (c ^ (r & 7)); }
-// V^T row d (128 bytes: 8 pieces of 8 keys) uses the K row swizzle: piece c at k_piece(d, c).
-constexpr int kImVe = kImVt + kPD * kKT * 2;        // int: e_tile, 2^e_tile > the tile's largest v norm
-constexpr int kImOnes = kImVe + 16;                 // row-sum operand: 4 dwords of 2^-e_tile (fp16 pair), 4 zero dwords
-constexpr int kImBytes = (kImOnes + 32 + 1023) / 1024 * 1024;  // whole 1 KB copies
-constexpr int kImChunks = kImBytes / 1024;
+// Tile image (bytes), the same in the workspace and in LDS: 64 K rows of 128 dims in the q
+// dtype (kw_piece: piece c holds dims 8c .. 8c+7), 128 V'^T rows of 64 fp16 keys (vw_piece),
+// then the tile's V exponent.
+constexpr int kImK = 0;
+constexpr int kImVt = kImK + kKT * kPD * 2;
+constexpr int kImVe = kImVt + kPD * kKT * 2;                 // int: e_tile, 2^e_tile > the tile's largest v norm
+constexpr int kImBytes = (kImVe + 4 + 1023) / 1024 * 1024;
+constexpr int kLdsK = kImVt + 16, kLdsV = kImVe - kImVt;       // LDS buffers: K rows and V exponent; V'^T rows
 
 // Keys of a sequence the attention may read: its length, bounded by the block
 // table's capacity and by the workspace's tile images.
@@ -160,17 +140,13 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(PrefillArgs a) {
         float vx = fmaxf(nvv, 0.f);
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) vx = fmaxf(vx, __shfl_xor(vx, o));
-        // 2^e_v > vx, clamped to [-14, 24] so that 2^-e_v is an fp16 (normal or denormal)
-        // value: the attention kernel's row-sum MFMA reads it.  Norms above 2^24 would
-        // overflow v' in fp16.
+        // 2^e_v > vx, clamped to [-14, 24]: norms below 2^-14 keep v' at their own scale, and
+        // norms above 2^24 would overflow v' in fp16.
         const int e_v = min(24, max(-14, (int)((__float_as_uint(vx) >> 23) & 0xffu) - 126));
         knorm[tid] = nkv;
         vnorm[tid] = nvv;
         if (tid == 0) {
             *reinterpret_cast<int *>(img + kImVe) = e_v;
-            const uint32_t w = pack_f16(ldexpf(1.f, -e_v), ldexpf(1.f, -e_v));
-            *reinterpret_cast<u32x4 *>(img + kImOnes) = u32x4{w, w, w, w};
-            *reinterpret_cast<u32x4 *>(img + kImOnes + 16) = u32x4{0u, 0u, 0u, 0u};
             vscale = ldexpf(1.f, -e_v);
         }
     }
@@ -203,19 +179,17 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(PrefillArgs a) {
             const uint32_t e1 = Elem<DT>::from_f32(opaque(ktab[(x >> (8 * j)) & 15u] * nrm));
             pr[j] = e0 | (e1 << 16);
         }
-        *reinterpret_cast<u32x4 *>(img + kImK + (dw >> 3) * (kKT * kKP) + k_piece(tk, dw & 7)) =
+        *reinterpret_cast<u32x4 *>(img + kImK + kw_piece(tk, dw)) =
             u32x4{pr[0], pr[1], pr[2], pr[3]};
     }
     // V'^T rows: v' = dtype(centroid * norm) * 2^-e_v (exact), rounded to fp16 (exact
-    // unless below fp16's normal range; |v'| < max|centroid|).  Key t = 16b + 4gg + i sits in piece
-    // 4 (b >> 1) + gg of its dim row, element 4 (b & 1) + i: thread (key quad,
-    // dword) writes 4 consecutive keys = 8 bytes.
+    // unless below fp16's normal range; |v'| < max|centroid|).  Thread (key quad, dword) writes 4 consecutive
+    // keys = 8 bytes per dim.
     {
         const int tq = tid & 15, dw = tid >> 4;  // key quad (4 consecutive keys), dword position
         const uint32_t(&x)[4] = xv;
         const int t0 = 4 * tq;
-        const int b = t0 >> 4, gg = (t0 >> 2) & 3;
-        const int piece = 4 * (b >> 1) + gg, elem_off = 8 * (b & 1);
+        const int piece = vw_quad_piece(tq), elem_off = vw_quad_byte(tq);
         float nv[4];
         const float vs = vscale;
 #pragma unroll
@@ -233,15 +207,25 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(PrefillArgs a) {
                     const float v = Elem<DT>::to_f32(Elem<DT>::from_f32(opaque(vtab[idx] * nv[i])));
                     e[i] = f32_to_f16_bits(v * vs);
                 }
-                *reinterpret_cast<uint2 *>(img + kImVt + k_piece(d, piece) + elem_off) =
+                *reinterpret_cast<uint2 *>(img + kImVt + vw_piece(d, piece) + elem_off) =
                     make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
             }
         }
     }
 }
 
+// ---- attention ----------------------------------------------------------------
+// What bounds it: vector issue and the matrix cores side by side.  A wave's tile is 32 MFMAs of
+// 32 cycles and about 115 vector instructions of 4 with 32 exponentials of 8 to 9; the MFMA unit
+// is busy 48 % of the time at 8 x 4096.  Two waves per SIMD (two workgroups of four waves per CU:
+// each has its own barriers, so one computes while the other waits): 64 accumulator, 64 score
+// and 32 query registers a lane.  Steps on 8 x 4096 causal, 32 / 8 heads, whole call: 16-position
+// waves at four per SIMD 1326 us; 32-position waves, one phase after the other 1337;
+// interleaved (step, below) 1375; R read from LDS instead of memory 1190; rotations without a
+// branch per dim and one rounding 1173.  Without the tile copies it takes 1082, without the tile
+// loop about 250 (copies of two tiles, rotations and stores).
 template <int DT>
-__global__ __launch_bounds__(1024) void prefill_attn_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_kernel(PrefillArgs a) {
     int qblk, h;
     int64_t seq;
     attn_work_item(qblk, h, seq);
@@ -250,145 +234,196 @@ __global__ __launch_bounds__(1024) void prefill_attn_kernel(PrefillArgs a) {
     const int L = a.seq_lens[seq];
     const int pos_base = L - T;  // position of query 0
     const int L_eff = visible_keys(a, seq);
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int nwaves = nthr >> 6;
-    // This wave's query head inside the GQA group (gh) and first query index (i0), and
-    // the workgroup's last query index.  Plain: wave = (gh, position group pg) of the
-    // workgroup's npg groups.  Flat (GQA groups whose G * npg waves would not spread
-    // evenly over a CU's four SIMDs, e.g. 7): the sequence's (position group, query
-    // head) units in position-group-major order, nwaves consecutive units per
-    // workgroup (at most two position groups when G < 8).
-    int gh, i0, last_i;
-    if (a.flat) {
-        const int units = T > 0 ? (T + kPQ - 1) / kPQ * a.G : 0;
-        const int f0 = qblk * nwaves;
-        if (f0 >= units) return;
-        const int f = f0 + wave;
-        gh = f % a.G;
-        i0 = f < units ? f / a.G * kPQ : T;  // units past the end: inactive
-        last_i = min(T, (min(f0 + nwaves, units) - 1) / a.G * kPQ + kPQ) - 1;
-    } else {
-        if (qblk * a.qb >= T || T <= 0) return;
-        gh = wave / a.npg;
-        const int pg = wave - gh * a.npg;  // 16-position group
-        i0 = qblk * a.qb + pg * kPQ;
-        last_i = min(T, (qblk + 1) * a.qb) - 1;
-    }
-    const int g = lane >> 4, col = lane & 15;
-    // this lane's operand pieces in a tile image: key col, pieces g and 4 + g; dim col, piece g
-    const int koff0 = k_piece(col, g), koff1 = k_piece(col, 4 + g);
-    const int ones_off = kImOnes + (col == 0 ? 0 : 16);  // the row-sum operand (MFMA row 0 = col 0)
-    const int hq = h * a.G + gh;
+    const int hh = lane >> 5, col = lane & 31;
+    // This wave's unit: (32-position group, query head of the GQA group) of the sequence and
+    // kv head, in position-group-major order; the workgroup's units span two position
+    // groups at most when G >= 4 (whatever G, the four SIMDs carry one wave each).
+    const int units = T > 0 ? (T + kPW - 1) / kPW * a.G : 0;
+    const int f0 = qblk * kWaves;
+    if (f0 >= units) return;
+    const int f = f0 + wave;
+    const int i0 = f < units ? f / a.G * kPW : T;  // first query index (units past the end: inactive)
+    const int last_i = min(T, (min(f0 + kWaves, units) - 1) / a.G * kPW + kPW) - 1;
+    const int hq = h * a.G + f % a.G;
     const bool wave_active = i0 < T;
     const int my_i = i0 + col;              // query index of this lane's column
     const int my_pos = pos_base + my_i;
 
-    // LDS: two tile-image buffers.
+    // LDS: two K buffers (K rows and the tile's V exponent) and two V'^T buffers.
     extern __shared__ __align__(16) uint8_t lds[];
+    uint8_t *const kbuf[2] = {lds, lds + kLdsK};
+    uint8_t *const vbuf[2] = {lds + 2 * kLdsK, lds + 2 * kLdsK + kLdsV};
+    float4 *const rot = reinterpret_cast<float4 *>(lds + 2 * (kLdsK + kLdsV));
 
-    // ---- key range: causal bound of the whole workgroup --------------------------
+    // ---- key range: causal bound of the whole workgroup and of this wave -----------
     const bool causal = a.causal;
     const int kv_end = causal ? min(L_eff, pos_base + last_i + 1) : L_eff;  // keys [0, kv_end) may be visible
-    const int n_tiles = (kv_end + kKT - 1) / kKT;
+    const int n_tiles = kv_end > 0 ? (kv_end + kKT - 1) / kKT : 0;
+    const int wv_end = causal ? min(kv_end, pos_base + i0 + kPW) : kv_end;
+    const int nw = wave_active && wv_end > 0 ? (wv_end + kKT - 1) / kKT : 0;  // tiles this wave takes part in
 
-    // Tile images of this (sequence, kv head), copied global -> LDS 1 KB per wave
-    // instruction into two buffers; tile t+1's copy runs while tile t is computed.
-    // Tiles 0 and 1 are issued first, so that their copies overlap the query
-    // operand's loads and arithmetic (the query operand uses no LDS).
+    // Tile images of this (sequence, kv head), copied global -> LDS 1 KB per wave instruction.
+    // The rotation of the query operand overlaps the first copies.
     const uint8_t *img0 = a.ws + ((int64_t)seq * a.H + h) * a.max_tiles * kImBytes;
     const uint32_t lds0 = lds_addr(lds);
-    auto issue_tile = [&](int t) {
-        const uint8_t *src = img0 + (int64_t)t * kImBytes;
-        const uint32_t dst = lds0 + (t & 1) * kImBytes;
-        for (int c = wave; c < kImChunks; c += nwaves) {
-            // wave-uniform operands of the copy (the compiler cannot prove it here)
-            const uint64_t s = reinterpret_cast<uint64_t>(src + c * 1024);
-            const uint32_t slo = __builtin_amdgcn_readfirstlane((uint32_t)s);
-            const uint32_t shi = __builtin_amdgcn_readfirstlane((uint32_t)(s >> 32));
-            const uint8_t *su = reinterpret_cast<const uint8_t *>(((uint64_t)shi << 32) | slo);
-            copy16(su, 16 * lane, __builtin_amdgcn_readfirstlane(dst + c * 1024));
+    auto copy_rows = [&](int t, int from, uint32_t dst_) {
+        const uint64_t s = reinterpret_cast<uint64_t>(img0 + (int64_t)t * kImBytes + from);
+        // wave-uniform operands of the copies (the compiler cannot prove it here)
+        const uint32_t slo = __builtin_amdgcn_readfirstlane((uint32_t)s);
+        const uint32_t shi = __builtin_amdgcn_readfirstlane((uint32_t)(s >> 32));
+        const uint8_t *src = reinterpret_cast<const uint8_t *>(((uint64_t)shi << 32) | slo);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(dst_);
+        static_assert(kImVt % (1024 * kWaves) == 0 && kImVe - kImVt == kImVt, "whole copies per wave");
+#pragma unroll
+        for (int u = 0; u < kImVt / (1024 * kWaves); ++u) {
+            const int c = u * kWaves + wave;
+            copy16(src + c * 1024, 16 * lane, dst + c * 1024);
         }
+        if (from == kImK && wave == 0 && lane == 0) copy16(src + kImVe, 0, dst + kImVt);  // the tile's V exponent
     };
-    if (n_tiles > 0) issue_tile(0);
-    if (n_tiles > 1) issue_tile(1);
-
-    // ---- Q^T operand (cols = this wave's 16 positions): q_rot rounded to the q dtype,
-    //      k-step s = dims 32s + 8g .. +7 ----
-    u32x4 qop[4];
-    if (wave_active) {
-        const int qi = i0 + col;
-        const bool qvalid = qi < T;
-        const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (qvalid ? qi : 0)) * a.q_st +
+    auto copy_k = [&](int t) { if (t < n_tiles) copy_rows(t, kImK, lds0 + (t & 1) * kLdsK); };
+    auto copy_v = [&](int t) { if (t < n_tiles) copy_rows(t, kImVt, lds0 + 2 * kLdsK + (t & 1) * kLdsV); };
+    // ---- Q^T operand (columns = this wave's 32 positions): q_rot rounded to the q dtype ----
+    // (the query row is loaded before the first copies go out: a wait of the compiler's for a
+    // load also waits for every copy issued before it)
+    u32x4 qop[8];
+    {
+        const bool qvalid = wave_active && my_i < T;
+        const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (qvalid ? my_i : 0)) * a.q_st +
                                (int64_t)hq * a.q_sh;
-#pragma unroll
-        for (int s_ = 0; s_ < 4; ++s_) {
-            const int base = 32 * s_ + 8 * g;
-            const uint4 rw = qvalid ? *reinterpret_cast<const uint4 *>(qrow + base) : make_uint4(0, 0, 0, 0);
-            const uint32_t w16[4] = {rw.x, rw.y, rw.z, rw.w};
-            float xin[8], qr[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) xin[k] = Elem<DT>::to_f32((w16[k >> 1] >> (16 * (k & 1))) & 0xffffu);
-            rotate_q8<DT>(xin, base, a.R, a.rot_block, qr);
-            uint32_t pk[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) pk[k] = Elem<DT>::from_f32(qr[2 * k]) | (Elem<DT>::from_f32(qr[2 * k + 1]) << 16);
-            qop[s_] = u32x4{pk[0], pk[1], pk[2], pk[3]};
-        }
+        wide_query_load(qop, qrow, qvalid, hh);
     }
+    load_rotation(rot, a.R, tid);
+    __syncthreads();
+#pragma unroll
+    for (int s_ = 0; s_ < 8; ++s_) asm volatile("" : "+v"(qop[s_]));  // (arrived)
+    copy_k(0);
+    copy_v(0);
+    copy_k(1);
+    copy_v(1);
+    wide_query<DT, false>(qop, rot, a.rot_block, hh);
 
-    AttnState st;
+    WideState st;
     st.init();
+    const WideOffsets wo(hh, col);
+    const float scale = a.score_scale;
+    f32x16 sa[2], sb[2];  // scores of an even and of an odd tile
+    float bias = 0.f;     // of the tile whose exponentials come next
+    int e_v = 0;          // its V exponent
+    // Mask of tile t's scores: at the diagonal and the end.
+    auto mask = [&](int t, f32x16 (&s)[2]) {
+        const int k0 = t * kKT, nk = min(kKT, kv_end - k0);
+        // every key of the tile visible to all 32 positions of this wave: no mask
+        if (!(nk == kKT && (!causal || k0 + kKT - 1 <= pos_base + i0)))
+            wide_mask(s, (causal ? min(k0 + nk, my_pos + 1) : k0 + nk) - (k0 + 4 * hh));
+    };
+    auto v_exponent = [&](const uint8_t *kt) {
+        return __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(kt + kImVt));
+    };
 
     // The first two tile images landed while the query operand was built.
-    if (n_tiles > 0) {
+    wait_copies<0>();
+    __syncthreads();
+    if (nw > 0) {
+        sa[0] = sa[1] = f32x16{};
+#pragma unroll
+        for (int f = 0; f < 16; ++f) sa[f & 1] = mfma32<DT>(wide_k(kbuf[0], wo, f >> 1, f & 1), qop[f >> 1], sa[f & 1]);
+        mask(0, sa);
+        e_v = v_exponent(kbuf[0]);
+        bias = wide_max(st, wide_lane_max(sa), scale, e_v);
+    }
+    // Before tile t: its V'^T and tile t+1's K have landed (for every wave), and every wave is
+    // done with tile t's K and tile t-1's V'^T, whose buffers are refilled.
+    auto turn = [&](int t) {
         wait_copies<0>();
         __syncthreads();
-    }
-
-    for (int ti = 0; ti < n_tiles; ++ti) {
-        const int k0 = ti * kKT;
-        const int nk = min(kKT, kv_end - k0);
-        const uint8_t *tb = lds + (ti & 1) * kImBytes;
-        if (ti >= 1 && ti + 1 < n_tiles) issue_tile(ti + 1);  // tile 1 went out with tile 0
-        // (every wave reaches the barrier at the end of the iteration)
-        if (wave_active && (!causal || k0 <= pos_base + i0 + kPQ - 1)) {  // else: tile above this wave's diagonal
-        // every key of the tile visible to all 16 positions of this wave: no mask
-        const bool full = nk == kKT && (!causal || k0 + kKT - 1 <= pos_base + i0);
-
-        // ---- S^T = K Q^T for 4 key blocks of 16 ----
-        float s[16];
+        copy_k(t + 2);
+        if (t > 0) copy_v(t + 1);
+    };
+    // Tile t (t % 2 == par): its exponentials and P V from sc, and tile t+1's scores into sn.
+    auto step = [&](auto par, int t, f32x16 (&sc)[2], f32x16 (&sn)[2]) {
+        constexpr int P = decltype(par)::value;
+        turn(t);
+        const uint8_t *kt = kbuf[P ^ 1], *vt = vbuf[P];
+        uint32_t pop[16];
+        float l = 0.f;
+        // Tile t+1's scores run on the matrix cores under tile t's exponentials, and tile t's
+        // P V under the search for tile t+1's maximum: an MFMA occupies its unit for 32 cycles
+        // and leaves the wave free to issue about 7 vector instructions (4 MFMAs and 28 FMAs
+        // of each of two waves on a SIMD: 130 ns interleaved, 164 one after the other, 110
+        // for the MFMAs alone).  The compiler neither interleaves them by itself nor reads
+        // operands far enough ahead of an LDS read's latency, so each slot below is
+        // fenced: an operand read, an MFMA, and a sixteenth of the vector work.
+        constexpr int kAhead = 5;  // operand reads in flight
+        constexpr int kPairsA = 10;
+        static_assert(kPairsA + 12 / 2 >= 16, "every weight before its product");
+        const WideOffsets o = wo.fresh();
+        u32x4 kf[16], vf[16];
+        int e_next = *reinterpret_cast<const int *>(kt + kImVt);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int f = 0; f < kAhead; ++f) kf[f] = wide_k(kt, o, f >> 1, f & 1);
+        sn[0] = sn[1] = f32x16{};
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {  // four k-steps of 32 dims (half ks / 2 of the key row)
-                const int ko = (ks >> 1) * (kKT * kKP) + 16 * b * kKP + ((ks & 1) ? koff1 : koff0);
-                const u32x4 kv = *reinterpret_cast<const u32x4 *>(tb + kImK + ko);
-                c = mfma_qk<DT>(kv, qop[ks], c);
+        for (int f = 0; f < 16; ++f) {
+            if (f + kAhead < 16) kf[f + kAhead] = wide_k(kt, o, (f + kAhead) >> 1, (f + kAhead) & 1);
+            else vf[f + kAhead - 16] = wide_v(vt, o, (f + kAhead - 16) >> 2, (f + kAhead - 16) & 3);
+            sn[f & 1] = mfma32<DT>(kf[f], qop[f >> 1], sn[f & 1]);
+            // pairs 0 .. 9 of the 16; the others run under the P V products that do not need them yet
+            if (kPairsA * (f + 1) / 16 > kPairsA * f / 16) {
+                wide_exp_pair(sc, kPairsA * f / 16, scale, bias, pop, l);
+                // (values used only after the mask's branch would be computed there)
+                asm volatile("" : "+v"(l), "+v"(pop[kPairsA * f / 16]));
             }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        e_next = __builtin_amdgcn_readfirstlane(e_next);
+        mask(t + 1, sn);
+        float lm = -INFINITY;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[4 * b + i] = c[i];
+        for (int f = 0; f < 16; ++f) {
+            if (f + kAhead < 16) vf[f + kAhead] = wide_v(vt, o, (f + kAhead) >> 2, (f + kAhead) & 3);
+            st.acc[f & 3] = mfma32<RQ_DTYPE_F16>(vf[f], wide_p(pop, f >> 2), st.acc[f & 3]);
+            lm = fmaxf(fmaxf(lm, sn[f >> 3][2 * (f & 7)]), sn[f >> 3][2 * (f & 7) + 1]);
+            if (f % 2 == 0 && kPairsA + f / 2 < 16) wide_exp_pair(sc, kPairsA + f / 2, scale, bias, pop, l);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (!full) {  // causal and tile-end mask: key < min(k0 + nk, position + 1)
-            const int lim = (causal ? min(k0 + nk, my_pos + 1) : k0 + nk) - (k0 + 4 * g);
+        wide_add_sum(st, l, e_v);
+        e_v = e_next;
+        bias = wide_max(st, lm, scale, e_v);
+    };
+    // This wave's last tile.
+    auto last = [&](const uint8_t *vt, const f32x16 (&sc)[2]) {
+        uint32_t pop[16];
+        float l = 0.f;
 #pragma unroll
-            for (int j = 0; j < 16; ++j) s[j] = (16 * (j >> 2) + (j & 3)) < lim ? s[j] : -INFINITY;
-        }
-        // ---- online softmax and O^T += V'^T P'^T ----
-        softmax_pv(st, s, a.score_scale, 1.f, *reinterpret_cast<const int *>(tb + kImVe), tb + kImVt, koff0, koff1,
-                   *reinterpret_cast<const u32x4 *>(tb + ones_off));
-        }
-        wait_copies<0>();  // the next tile's image has landed
-        __syncthreads();   // ... for every wave; this buffer is refilled next
+        for (int i = 0; i < 16; ++i) wide_exp_pair(sc, i, scale, bias, pop, l);
+        wide_add_sum(st, l, e_v);
+#pragma unroll
+        for (int f = 0; f < 16; ++f)
+            st.acc[f & 3] = mfma32<RQ_DTYPE_F16>(wide_v(vt, wo, f >> 2, f & 3), wide_p(pop, f >> 2), st.acc[f & 3]);
+    };
+    int t = 0;
+    while (t + 1 < nw) {
+        step(std::integral_constant<int, 0>{}, t++, sa, sb);
+        if (t + 1 >= nw) break;
+        step(std::integral_constant<int, 1>{}, t++, sb, sa);
     }
+    if (nw > 0) {
+        turn(t);
+        if (t & 1) last(vbuf[1], sb);
+        else last(vbuf[0], sa);
+        ++t;
+    }
+    for (; t < n_tiles; ++t) turn(t);  // tiles above this wave's diagonal: only their copies and barriers
     if (!wave_active) return;
 
     // ---- epilogue: normalise, round to the q dtype, rotate back by R, round ----
-    const float inv_l = attn_inv_l(st);
-    if (i0 + col >= T) return;
-    uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + i0 + col) * a.o_st + (int64_t)hq * a.o_sh;
-    store_rotated<DT>(st, inv_l, orow, a.R, a.rot_block, g);
+    const bool ovalid = my_i < T;
+    uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + (ovalid ? my_i : 0)) * a.o_st + (int64_t)hq * a.o_sh;
+    wide_store<DT>(st, ovalid, orow, rot, a.rot_block, hh);
 }
 
 template <int DT>
@@ -398,11 +433,11 @@ static void launch_pack(const PrefillArgs &a, int64_t num_seqs, hipStream_t st) 
 }
 
 template <int DT>
-static void launch_attn(const PrefillArgs &a, int64_t num_seqs, int64_t max_q_len, int nwaves, hipStream_t st) {
-    const size_t lds = 2 * (size_t)kImBytes;
-    const int64_t nx = a.flat ? ((max_q_len + kPQ - 1) / kPQ * a.G + nwaves - 1) / nwaves : (max_q_len + a.qb - 1) / a.qb;
+static void launch_attn(const PrefillArgs &a, int64_t num_seqs, int64_t max_q_len, hipStream_t st) {
+    const size_t lds = 2 * (size_t)(kLdsK + kLdsV) + kRotBytes;
+    const int64_t nx = ((max_q_len + kPW - 1) / kPW * a.G + kWaves - 1) / kWaves;
     dim3 grid((unsigned)nx, (unsigned)a.H, (unsigned)num_seqs);
-    hipLaunchKernelGGL((prefill_attn_kernel<DT>), grid, dim3(64 * nwaves), lds, st, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<DT>), grid, dim3(64 * kWaves), lds, st, a);
 }
 
 static int64_t prefill_tiles(int64_t max_seq_len) { return (max_seq_len + kKT - 1) / kKT; }
@@ -482,27 +517,19 @@ int prefill_call(bool fused, int causal, const void *q, int32_t dtype, int64_t t
     a.rot_block = rot_block;
     a.score_scale = sm_scale * kLog2eP;
     a.causal = causal != 0;
-    a.npg = std::max(1, 8 / a.G);
-    a.qb = kPQ * a.npg;
-    // GQA groups of 3, 5, 6 or 7 query heads: G * npg waves (6, 5, 6, 7) per workgroup
-    // would load a CU's four SIMDs unevenly (two 7-wave workgroups: 4, 4, 3, 3 waves,
-    // and each tile's barrier paces a workgroup by its busiest SIMD); they take
-    // workgroups of 8 waves over the flattened (position group, query head) units.
-    a.flat = a.G < 8 && (a.G * a.npg) % 4 != 0;
     a.max_tiles = prefill_tiles(max_seq_len);
     a.ws = static_cast<uint8_t *>(workspace);
     a.out = out;
     a.o_st = out_stride_tok;
     a.o_sh = out_stride_head;
-    const int nwaves = a.flat ? 8 : a.G * a.npg;
     hipStream_t st = (hipStream_t)stream;
     const bool bf = dtype == RQ_DTYPE_BF16;
     if (bf) launch_pack<RQ_DTYPE_BF16>(a, num_seqs, st);
     else launch_pack<RQ_DTYPE_F16>(a, num_seqs, st);
     int rc = check_launch("prefill_pack_kernel");
     if (rc) return rc;
-    if (bf) launch_attn<RQ_DTYPE_BF16>(a, num_seqs, max_q_len, nwaves, st);
-    else launch_attn<RQ_DTYPE_F16>(a, num_seqs, max_q_len, nwaves, st);
+    if (bf) launch_attn<RQ_DTYPE_BF16>(a, num_seqs, max_q_len, st);
+    else launch_attn<RQ_DTYPE_F16>(a, num_seqs, max_q_len, st);
     return check_launch("prefill_attn_kernel");
 }
 

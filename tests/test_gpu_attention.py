@@ -141,6 +141,17 @@ def test_attention_single_key_closed_form(entry):
     assert np.abs(got - exp).max() <= 1e-2 * max(1.0, float(np.abs(exp).max()))
 
 
+@pytest.mark.parametrize("H,HQ,mode,dtype", [(2, 6, "planar", torch.bfloat16), (1, 5, "iso", torch.float16),
+                                             (1, 1, "iso", torch.bfloat16)])
+def test_attention_position_group_edges(H, HQ, mode, dtype, entry):
+    """Query lengths around the 32-position groups of a wave, alone and behind prefixes that put the
+    causal diagonal at every offset of a 64-key tile's halves; workgroups of 4 (position group, head)
+    units that straddle position groups (3, 5 heads) or hold four of them (1 head)."""
+    q_lens = [31, 32, 33, 64, 95, 97, 129]
+    ctx = [q + pre for q, pre in zip(q_lens, [0, 31, 33, 1, 64, 30, 255])]
+    check(attn_case(74 + HQ, q_lens, ctx, H, HQ, Params(mode, 4, 3), dtype=dtype), f"groups-{HQ}", entry=entry)
+
+
 def test_attention_graph_replay():
     """The call captured in a HIP graph: each replay, after the eager work between
     replays (new q and context lengths written into the captured buffers), equals
