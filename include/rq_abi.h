@@ -375,6 +375,38 @@ int rq_paged_prefill(const void *q, int32_t dtype, int64_t total_q, int32_t num_
  * writes a decompressed copy of every referenced page instead. */
 int64_t rq_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads, int64_t max_seq_len);
 
+/*
+ * rq_paged_prefill for queries of a few tokens (drafts being verified), on the
+ * kernels of rq_fused_decode: the (token, query head) pairs of a kv head share its
+ * stream of packed keys, up to 16 pairs at a time, so nothing is unpacked to memory
+ * and the batch's keys are split over the whole GPU.  Arithmetic of the decode
+ * kernels (K and V in the q dtype, exact products, fp32 sums).
+ *
+ * Replaces the same reference code as rq_paged_attention (rq_backend.py:937-1036).
+ * Arguments as for rq_paged_prefill, with rq_fused_decode's restrictions: 8 or 16
+ * centroids, cache slots, centroids and rotation 16-byte aligned, at most 64 kv heads.
+ * workspace: rq_short_attention_workspace_bytes() bytes, 16-byte aligned, no
+ * initialisation needed; that is 0 for shapes the call does not take (a query's tokens
+ * and heads need more than 4 groups of 16 columns, e.g. more than 16 tokens of 4 heads,
+ * or too many sequences).  Launch sizes depend on host arguments only.
+ */
+int64_t rq_short_attention_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                           int64_t max_q_len, int64_t max_seq_len);
+int rq_short_attention(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,
+                       int64_t q_stride_tok, int64_t q_stride_head,
+                       const int32_t *cu_seqlens_q, int64_t num_seqs, int64_t max_q_len, int32_t causal,
+                       const uint8_t *kv_cache, int64_t num_blocks, int32_t block_size,
+                       int64_t stride_block, int64_t stride_token,
+                       int32_t num_kv_heads, int32_t head_dim, int32_t index_layout,
+                       const int32_t *block_table, int64_t max_blocks, int64_t bt_stride_seq,
+                       const int32_t *seq_lens, int64_t max_seq_len,
+                       const float *k_centroids, int32_t n_k_centroids,
+                       const float *v_centroids, int32_t n_v_centroids,
+                       const float *rotation, int32_t rot_block, float sm_scale,
+                       void *out, int64_t out_stride_tok, int64_t out_stride_head,
+                       void *workspace, int64_t workspace_bytes,
+                       void *stream);
+
 #ifdef __cplusplus
 }
 #endif

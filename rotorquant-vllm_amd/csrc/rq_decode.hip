@@ -22,6 +22,11 @@
 //   * decode_merge_kernel: log-sum-exp over a sequence's partials, rounding and
 //     the rotation back by R.
 //
+// rq_short_attention runs the same kernels on sequences of a few query tokens each
+// (drafts being verified): the MFMA columns of a kv head, which hold its query heads
+// for one token, then hold the (token, query head) pairs of up to 16 / G tokens, and a
+// sequence with more tokens appears several times (column groups) in the tile list.
+//
 // MFMA operand layout used below (16x16x32, wave64, lane l, g = l / 16):
 //   A (16 x 32): lane holds row l % 16, k = 8g .. 8g+7   (4 dwords of 2 x 16-bit)
 //   B (32 x 16): lane holds col l % 16, k = 8g .. 8g+7
@@ -58,6 +63,9 @@ constexpr int kTile = 32;        // tokens per inner iteration
 constexpr int kMaxWaves = 8;     // kv heads (= waves) per workgroup
 constexpr int kMaxKvHeads = 64;
 constexpr float kLog2e = 1.4426950408889634f;
+// Running max before a column has seen a key: finite, so that a tile whose scores are all
+// -inf for a column (a query token that does not reach the tile) leaves it and gives p = 0.
+constexpr float kNoMax = -3.0e38f;
 
 template <int DT>
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -169,6 +177,10 @@ struct DecodeArgs {
     int block_size;
     int bs_shift;       // log2(block_size), or -1 when block_size is not a power of two
     int H, G, HQ;
+    int GC, HC;         // columns per kv head (G x tokens of a column group; <= 16) and H * GC
+    const int32_t *cu_q;  // short queries: query starts per sequence (nullptr: one token per sequence)
+    int tpg, vg;        // tokens per column group, column groups per sequence
+    int causal;         // short queries: token i sees the keys up to its own position only
     const int32_t *bt;
     int64_t bt_ss;
     int64_t max_blocks;
@@ -191,9 +203,9 @@ struct DecodeArgs {
     int *tile_prefix;   // [seq][2]: first workgroup whose range covers the sequence, number of such workgroups
     int *n_tiles_total;
     uint64_t *split_m;  // M of the range split (prep kernel)
-    uint32_t *qops;     // [seq][H][16 cols][4 g][4 chunks][4 dwords]: q-dtype query operands (cols < G written)
-    float *part_acc;    // [slot][HQ][D], slot = workgroup + seq
-    float *part_ml;     // [slot][HQ][2]
+    uint32_t *qops;     // [seq][H][16 cols][4 g][4 chunks][4 dwords]: q-dtype query operands (cols < GC written)
+    float *part_acc;    // [slot][HC][D], slot = workgroup + seq
+    float *part_ml;     // [slot][HC][2]
     void *out;
     int64_t o_ss, o_sh;
 };
@@ -215,13 +227,45 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// q_rot = q R^T of the G query heads of (seq, kv head h), rounded to the query
+// What the tile list calls a sequence ("entry"): a sequence, or with short queries one
+// column group of one -- tokens i0 .. i0 + ntok - 1 of sequence b, column c being token
+// i0 + c / G, query head c % G of the kv head.
+struct Entry {
+    int64_t b, row0;  // sequence; query (and output) row of the entry's first token
+    int ntok;         // <= 0: a group past the sequence's tokens
+};
+template <bool SHORT>
+__device__ __forceinline__ Entry entry_of(const DecodeArgs &a, int64_t e) {
+    if constexpr (!SHORT) return Entry{e, e, 1};
+    const int b = (int)e / a.vg, i0 = ((int)e - b * a.vg) * a.tpg;
+    const int q0 = a.cu_q[b];
+    return Entry{b, q0 + i0, min(a.tpg, a.cu_q[b + 1] - q0 - i0)};
+}
+// Keys of an entry: those its last token sees.
+template <bool SHORT>
+__device__ __forceinline__ int entry_len(const DecodeArgs &a, int64_t e) {
+    if constexpr (!SHORT) return min(a.seq_lens[e], a.max_len);
+    const int b = (int)e / a.vg, i0 = ((int)e - b * a.vg) * a.tpg;
+    const int T = a.cu_q[b + 1] - a.cu_q[b], L = a.seq_lens[b];
+    if (i0 >= T) return 0;
+    const int Le = min(L, a.max_len);
+    return a.causal ? min(Le, L - T + min(T, i0 + a.tpg)) : Le;
+}
+// Of those (L = entry_len), the keys its first token sees; may be <= 0.
+template <bool SHORT>
+__device__ __forceinline__ int entry_first(const DecodeArgs &a, int64_t e, int L) {
+    if (!SHORT || !a.causal) return L;
+    const int b = (int)e / a.vg, i0 = ((int)e - b * a.vg) * a.tpg;
+    return min(L, a.seq_lens[b] - (a.cu_q[b + 1] - a.cu_q[b]) + i0 + 1);
+}
+
+// q_rot = q R^T of the GC columns of (entry, kv head h), rounded to the query
 // dtype (fused_paged_rq_decode.py:271), as the Q^T MFMA operand in that dtype:
 // lane (g, col) holds for dim chunk c the dims 32g + 8c + {0,2,4,6,1,3,5,7} of
-// query head col (zero for col >= G).
-// wq: this wave's LDS scratch of G * 128 16-bit values.
-template <int DT>
-__device__ __forceinline__ void query_operand(const DecodeArgs &a, int64_t seq, int h, uint16_t *wq, u32x4 (&qop)[4]) {
+// column col (zero for col >= GC; columns past the entry's last token repeat it).
+// wq: this wave's LDS scratch of GC * 128 16-bit values.
+template <int DT, bool SHORT>
+__device__ __forceinline__ void query_operand(const DecodeArgs &a, const Entry &en, int h, uint16_t *wq, u32x4 (&qop)[4]) {
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, col = lane & 15;
     {
@@ -242,12 +286,22 @@ __device__ __forceinline__ void query_operand(const DecodeArgs &a, int64_t seq, 
             r0[0] = x.x, r0[1] = x.y, r0[2] = 0.f, r0[3] = 0.f;
             r1[0] = y.x, r1[1] = y.y, r1[2] = 0.f, r1[3] = 0.f;
         }
-        const uint16_t *qbase = reinterpret_cast<const uint16_t *>(a.q) + seq * a.q_ss + (int64_t)(h * a.G) * a.q_sh + k0;
-        for (int qh0 = 0; qh0 < a.G; qh0 += 4) {
+        const uint16_t *qbase = reinterpret_cast<const uint16_t *>(a.q) + en.row0 * a.q_ss + (int64_t)(h * a.G) * a.q_sh + k0;
+        [[maybe_unused]] int tok = 0, gh = 0;  // of column qh0 + u
+        for (int qh0 = 0; qh0 < a.GC; qh0 += 4) {
             uint2 raw[4];
     #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const uint16_t *qp = qbase + (int64_t)min(qh0 + u, a.G - 1) * a.q_sh;
+                const uint16_t *qp = qbase;
+                if constexpr (!SHORT) {
+                    qp += (int64_t)min(qh0 + u, a.G - 1) * a.q_sh;
+                } else {
+                    qp += (int64_t)min(tok, en.ntok - 1) * a.q_ss + (int64_t)gh * a.q_sh;
+                    if (++gh == a.G) {
+                        gh = 0;
+                        ++tok;
+                    }
+                }
                 raw[u] = rb == 4 ? *reinterpret_cast<const uint2 *>(qp) : make_uint2(*reinterpret_cast<const uint32_t *>(qp), 0u);
             }
     #pragma unroll
@@ -262,7 +316,7 @@ __device__ __forceinline__ void query_operand(const DecodeArgs &a, int64_t seq, 
                         acc1 = __builtin_fmaf(x, r1[i], acc1);
                     }
                 }
-                if (qh0 + u < a.G)
+                if (qh0 + u < a.GC)
                     reinterpret_cast<uint32_t *>(wq + (qh0 + u) * kD)[lane] =
                         Elem<DT>::from_f32(acc0) | (Elem<DT>::from_f32(acc1) << 16);
             }
@@ -272,7 +326,7 @@ __device__ __forceinline__ void query_operand(const DecodeArgs &a, int64_t seq, 
     #pragma unroll
     for (int c = 0; c < 4; ++c) {
         // w: dims 8c' .. 8c'+7 (c' = 4g + c) as 16-bit pairs (d0 d1) (d2 d3) (d4 d5) (d6 d7)
-        const uint4 w = col < a.G ? *reinterpret_cast<const uint4 *>(wq + col * kD + 32 * g + 8 * c)
+        const uint4 w = col < a.GC ? *reinterpret_cast<const uint4 *>(wq + col * kD + 32 * g + 8 * c)
                                   : make_uint4(0, 0, 0, 0);
         qop[c] = u32x4{perm(w.y, w.x, 0x05040100u), perm(w.w, w.z, 0x05040100u),   // (d0 d2) (d4 d6)
                        perm(w.y, w.x, 0x07060302u), perm(w.w, w.z, 0x07060302u)};  // (d1 d3) (d5 d7)
@@ -296,7 +350,9 @@ __device__ __forceinline__ void wait_copies_upto(int n) {
 // Tile descriptor: one 32-token tile of one sequence, written by the prep kernel
 // and read by the decode workgroup that owns the tile.
 struct TileDesc {
-    int32_t seq, tile, valid, pad;  // sequence, tile index inside it, tokens in the tile (1..32)
+    int32_t seq, tile, valid;       // entry, tile index inside it, tokens in the tile (1..32)
+    int32_t lim;                    // tokens of the tile that the entry's first query token sees (each
+                                    // following token one more, up to valid); valid when all see the tile
     uint64_t off[kTile];            // byte offset of each token's slot (0 past `valid`)
 };
 static_assert(sizeof(TileDesc) == 16 + 8 * kTile, "TileDesc layout");
@@ -354,8 +410,9 @@ __device__ __forceinline__ int range_start(const RangeSplit r, int w) {
 }
 
 
-__device__ __forceinline__ int seq_tiles(const DecodeArgs &a, int64_t b) {
-    const int L = min(a.seq_lens[b], a.max_len);
+template <bool SHORT>
+__device__ __forceinline__ int seq_tiles(const DecodeArgs &a, int64_t e) {
+    const int L = entry_len<SHORT>(a, e);
     return L > 0 ? (L + kTile - 1) / kTile : 0;
 }
 
@@ -369,7 +426,7 @@ __device__ __forceinline__ int seq_tiles(const DecodeArgs &a, int64_t b) {
 //   * tile_prefix[seq] = the first decode workgroup whose range covers the
 //     sequence and the number of such workgroups (for the merge); the last
 //     sequence also stores the total tile count and the range-split multiplier.
-template <int DT>
+template <int DT, bool SHORT>
 __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
     const int64_t seq = blockIdx.x;
     const int y = blockIdx.y;
@@ -379,14 +436,15 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
     extern __shared__ __align__(16) uint8_t prep_lds[];  // query staging, 16 x kD 16-bit values per wave
     __shared__ int part[2 * kMaxWaves];
     // a descriptor workgroup past the end of its sequence's tokens has nothing to do
-    if (y >= 1 && 4 * (y - 1) * (int)blockDim.x >= seq_tiles(a, seq) * kTile) return;
-    if (y == 0) {
+    if (y >= 1 && 4 * (y - 1) * (int)blockDim.x >= seq_tiles<SHORT>(a, seq) * kTile) return;
+    const Entry en = entry_of<SHORT>(a, seq);
+    if (y == 0 && en.ntok > 0) {
         for (int h = wave; h < a.H; h += nw) {
             u32x4 qop[4];
-            query_operand<DT>(a, seq, h, reinterpret_cast<uint16_t *>(prep_lds) + wave * 16 * kD, qop);
+            query_operand<DT, SHORT>(a, en, h, reinterpret_cast<uint16_t *>(prep_lds) + wave * 16 * kD, qop);
             const int g = lane >> 4, col = lane & 15;
             uint4 *dst = reinterpret_cast<uint4 *>(a.qops + ((seq * a.H + h) * 16 + col) * 64 + g * 16);
-            if (col < a.G) {
+            if (col < a.GC) {
     #pragma unroll
                 for (int c = 0; c < 4; ++c) dst[c] = make_uint4(qop[c].x, qop[c].y, qop[c].z, qop[c].w);
             }
@@ -395,7 +453,7 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
     // tiles before this sequence (prefix) and in all sequences (NT)
     int cnt = 0, tot = 0;
     for (int64_t b = threadIdx.x; b < gridDim.x; b += blockDim.x) {
-        const int nb = seq_tiles(a, b);
+        const int nb = seq_tiles<SHORT>(a, b);
         cnt += b < seq ? nb : 0;
         tot += nb;
     }
@@ -413,8 +471,9 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
         prefix += part[w];
         NT += part[kMaxWaves + w];
     }
-    const int n = seq_tiles(a, seq);
-    const int L = min(a.seq_lens[seq], a.max_len);
+    const int n = seq_tiles<SHORT>(a, seq);
+    const int L = entry_len<SHORT>(a, seq);
+    const int L0 = entry_first<SHORT>(a, seq, L);
     if (y == 0 && wave == 0) {
         // The decode workgroups whose ranges cover this sequence (for the merge):
         // the owner of tile t is the number of w in [1, G) with range_start(w) <= t
@@ -448,7 +507,7 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
         }
     }
     if (y == 0) return;  // the query operands above are this workgroup's share
-    const int32_t *bt_row = a.bt + seq * a.bt_ss;
+    const int32_t *bt_row = a.bt + en.b * a.bt_ss;
     // four consecutive tokens per thread and step (block-table loads issued together),
     // on the workgroups y = 1 .. gridDim.y - 1
     const int ny = gridDim.y - 1;
@@ -476,7 +535,7 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
             d->seq = (int32_t)seq;
             d->tile = j0 / kTile;
             d->valid = min(kTile, L - j0);
-            d->pad = 0;
+            d->lim = min(kTile, L0 - j0);
         }
     }
 }
@@ -545,11 +604,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
 
     extern __shared__ __align__(16) uint8_t lds[];
     const TileDesc *const ring = reinterpret_cast<const TileDesc *>(lds + NS * stage_bytes);
-    // Query operand slot: per wave, its kv head's G columns (256 bytes each); then
+    // Query operand slot: per wave, its kv head's GC columns (256 bytes each); then
     // the K and V codebooks (16 floats each, zero-padded).
-    const int G = a.G;
+    const int GC = a.GC;
     uint8_t *const qarea = lds + NS * stage_bytes + RING * sizeof(TileDesc);
-    float *const cbarea = reinterpret_cast<float *>(qarea + hpw * G * 256);
+    float *const cbarea = reinterpret_cast<float *>(qarea + hpw * GC * 256);
 
     // Byte offset in a stage of byte b of 16-byte piece p of token t (pieces: K indices
     // of the hpw heads, 4 per head, then V indices; nibble layouts).  swz(t) = (t >> 1) & 7
@@ -634,14 +693,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
     };
 
     // Query operand of sequence s -> the query slot (each wave its own kv head):
-    // ceil(G / 4) 16-byte copies per wave.
+    // ceil(GC / 4) 16-byte copies per wave.
     auto issue_q = [&](int s) {
         const uint8_t *src = reinterpret_cast<const uint8_t *>(a.qops) + ((int64_t)s * a.H + h0 + wave) * 16 * 256;
-        const uint32_t dst = lds_addr(qarea + wave * G * 256);
+        const uint32_t dst = lds_addr(qarea + wave * GC * 256);
         const uint32_t l16 = 16u * lane_now();
-        for (int j = 0; j < G * 256; j += 1024)
-            if (j + l16 < (uint32_t)(G * 256)) copy16(src, j + l16, dst + j);
-        return (G + 3) / 4;
+        for (int j = 0; j < GC * 256; j += 1024)
+            if (j + l16 < (uint32_t)(GC * 256)) copy16(src, j + l16, dst + j);
+        return (GC + 3) / 4;
     };
 
     // The codebook loads are compiler-visible: issued before the descriptor copies
@@ -671,16 +730,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
     const float sc = a.score_scale;
     auto begin_segment = [&]() {
         const uint32_t ln = lane_now(), lc = ln & 15;  // rebuilt here, not kept live across the loop
-        const uint32_t qc = WIDE ? lc : (lc & 7);      // query head of this lane's column
-        const uint4 *src = reinterpret_cast<const uint4 *>(qarea + wave * G * 256 + qc * 256 + (ln >> 4) * 64);
+        const uint32_t qc = WIDE ? lc : (lc & 7);      // this lane's column
+        const uint4 *src = reinterpret_cast<const uint4 *>(qarea + wave * GC * 256 + qc * 256 + (ln >> 4) * 64);
     #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const uint4 v = (int)qc < G ? src[c] : make_uint4(0, 0, 0, 0);
+            const uint4 v = (int)qc < GC ? src[c] : make_uint4(0, 0, 0, 0);
             qop[c] = u32x4{v.x, v.y, v.z, v.w};
         }
     #pragma unroll
         for (int m = 0; m < NACC; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-        m_run = -INFINITY;  // running max (log2 domain) for this lane's query head
+        m_run = kNoMax;     // running max (log2 domain) for this lane's column
         l_run = 0.f;        // this lane's partial sum of p
         // bf16: the V operand is V * 2^-e_run <= max|c| (fp16); starting at 2^-64 keeps
         // tiny norms representable until the first tile raises it.
@@ -695,8 +754,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         const float lsum = rows_sum(l_run);
         const uint32_t ln = lane_now(), lc = ln & 15, lg = ln >> 4;
         const uint32_t qc = WIDE ? lc : (lc & 7);
-        if ((int)qc < a.G) {
-            const int64_t slot = (int64_t)(w + seq) * a.HQ + (h0 + wave) * a.G;  // uniform: query head h*G of the slot
+        if ((int)qc < a.GC) {
+            const int64_t slot = (int64_t)(w + seq) * a.HC + (h0 + wave) * a.GC;  // uniform: column h*GC of the slot
             uint8_t *pa = reinterpret_cast<uint8_t *>(a.part_acc + slot * kD);
             uint8_t *pm = reinterpret_cast<uint8_t *>(a.part_ml + slot * 2);
             const uint32_t hoff = qc * kD * 4;
@@ -753,6 +812,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
 
         const int tseq = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].seq);
         const int valid = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].valid);
+        const int qlim = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].lim);
         if (tseq != seq) {  // a new sequence starts at this tile
             if (seq >= 0) end_segment();
             seq = tseq;
@@ -922,9 +982,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         // The score scale sc > 0 enters the exponent's fma (and the max, which it
         // commutes with).
         float s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-        if (valid < kTile) {
-            const int vv = opaque_s(valid);
-            const int g4 = 4 * (int)(lane_now() >> 4);
+        if (qlim < kTile) {
+            // (this lane's query token of the entry: its column / G)
+            const uint32_t ln = lane_now();
+            const int tok = (int)((WIDE ? ln & 15u : ln & 7u) / (uint32_t)opaque_s(a.G));
+            const int vv = min(valid, opaque_s(qlim) + tok);
+            const int g4 = 4 * (int)(ln >> 4);
     #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int tt = i < 4 ? g4 + i : 12 + g4 + i;
@@ -939,7 +1002,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         // the result does not depend on when the rescale happens.
         if (__any(tmax > m_run + 8.f)) {
             const float m_new = fmaxf(m_run, tmax);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // m_run = -inf on the first tile -> 0
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // m_run = kNoMax on the first tile -> 0
     #pragma unroll
             for (int m = 0; m < NACC; ++m) acc[m] *= alpha;
             l_run *= alpha;
@@ -1003,7 +1066,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
 // workgroup share one query head, wave i taking segment passes i, i + kSplit, ...,
 // and wave 0 combines their (max, sum, accumulator) states through LDS -- one
 // round of loads instead of a chain of passes, on kSplit times as many waves.
-template <int DT, int kMergePass, int kSplit>
+template <int DT, int kMergePass, int kSplit, bool SHORT>
 __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     static_assert(kSplit == 1 || kSplit == 4, "one wave per head, or four (the 256-thread block)");
     const int64_t seq = blockIdx.y;
@@ -1012,7 +1075,17 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     const int share = kSplit == 1 ? 0 : wave;  // first segment pass of this wave
     __shared__ float orot_all[4][kD];
     float *orot = orot_all[wave];
-    if (hq >= a.HQ) return;  // (kSplit > 1: the whole workgroup or none of it)
+    if (hq >= (SHORT ? a.HC : a.HQ)) return;  // (kSplit > 1: the whole workgroup or none of it)
+    int64_t orow = seq;  // output row and head of this column
+    int ohead = hq;
+    if constexpr (SHORT) {
+        const Entry en = entry_of<SHORT>(a, seq);
+        const int hkv = hq / a.GC, hcol = hq - hkv * a.GC;
+        const int tok = hcol / a.G;  // query token of the entry
+        if (tok >= en.ntok) return;  // (likewise)
+        orow = en.row0 + tok;
+        ohead = hkv * a.G + (hcol - tok * a.G);
+    }
     // R entries for this lane's two output dims (issued first; independent of the partials)
     float rr[2][4];
     #pragma unroll
@@ -1031,13 +1104,13 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     // the prep kernel for every sequence), and used only when the sequence has tiles.
     const int tp_lo = a.tile_prefix[2 * seq], tp_n = a.tile_prefix[2 * seq + 1];
     const int ntt = *a.n_tiles_total;
-    const int n = seq_tiles(a, seq);
+    const int n = seq_tiles<SHORT>(a, seq);
     const int w_lo = n > 0 ? tp_lo : 0, nch = n > 0 ? tp_n : 0;
     const RangeSplit rsp = make_split(a, ntt);
     auto has_tiles = [rsp](int w) { return range_start(rsp, w + 1) > range_start(rsp, w); };
-    const float *ml = a.part_ml + (w_lo + seq) * (int64_t)a.HQ * 2 + hq * 2;
-    const float *pa = a.part_acc + (w_lo + seq) * (int64_t)a.HQ * kD + hq * kD;
-    const int64_t cs_ml = (int64_t)a.HQ * 2, cs_acc = (int64_t)a.HQ * kD;
+    const float *ml = a.part_ml + (w_lo + seq) * (int64_t)(SHORT ? a.HC : a.HQ) * 2 + hq * 2;
+    const float *pa = a.part_acc + (w_lo + seq) * (int64_t)(SHORT ? a.HC : a.HQ) * kD + hq * kD;
+    const int64_t cs_ml = (int64_t)(SHORT ? a.HC : a.HQ) * 2, cs_acc = (int64_t)(SHORT ? a.HC : a.HQ) * kD;
     float lsum = 0.f, o0 = 0.f, o1 = 0.f, M = -INFINITY;
     for (int c0 = share * kMergePass; c0 < nch; c0 += kSplit * kMergePass) {
         // lane c (< kMergePass) loads segment c0 + c's (m, l); every lane loads its two
@@ -1098,11 +1171,11 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
             o1 += f * x.y;
         }
     }
-    const float inv = nch > 0 ? 1.f / lsum : 0.f;  // empty context -> zeros (reference: acc 0, l 1)
+    const float inv = nch > 0 && lsum > 0.f ? 1.f / lsum : 0.f;  // no key seen -> zeros (reference: acc 0, l 1)
     orot[2 * lane] = Elem<DT>::to_f32(Elem<DT>::from_f32(o0 * inv));
     orot[2 * lane + 1] = Elem<DT>::to_f32(Elem<DT>::from_f32(o1 * inv));
     __builtin_amdgcn_wave_barrier();
-    uint16_t *dst = reinterpret_cast<uint16_t *>(a.out) + seq * a.o_ss + (int64_t)hq * a.o_sh;
+    uint16_t *dst = reinterpret_cast<uint16_t *>(a.out) + orow * a.o_ss + (int64_t)ohead * a.o_sh;
     uint32_t packed = 0;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -1148,7 +1221,7 @@ static int decode_per_cu(const DecodeArgs &a, size_t lds) {
             hipSuccess ||
         nb <= 0)
         nb = 1;
-    nb = std::min(nb, decode_wg_cap(a.hpw, a.HQ));
+    nb = std::min(nb, decode_wg_cap(a.hpw, a.HC));
     std::lock_guard<std::mutex> lock(mu);
     for (auto &e : cache[dev]) {
         if (e[0] == (int)lds && e[1] > 0) break;  // another caller stored it meanwhile
@@ -1211,7 +1284,7 @@ static void launch_decode_w(DecodeArgs &a, size_t lds, hipStream_t st, bool conf
 
 template <int DT, int KB, int VB, bool D3 = false>
 static void launch_decode(DecodeArgs &a, size_t lds, hipStream_t st, bool configure, KernelEvents ev) {
-    if (a.G > 8) launch_decode_w<DT, KB, VB, D3, true>(a, lds, st, configure, ev);
+    if (a.GC > 8) launch_decode_w<DT, KB, VB, D3, true>(a, lds, st, configure, ev);
     else launch_decode_w<DT, KB, VB, D3, false>(a, lds, st, configure, ev);
 }
 
@@ -1252,6 +1325,12 @@ extern "C" int64_t rq_fused_decode_workspace_bytes(int64_t num_seqs, int32_t num
     return DecodeWorkspace(num_seqs, num_q_heads, std::max<int64_t>(max_seq_len, 1)).total;
 }
 
+// rq_short_attention's queries: cu_q per sequence, column groups of tpg tokens, vg per sequence.
+struct ShortQueries {
+    const int32_t *cu_q = nullptr;
+    int tpg = 1, vg = 1, causal = 0;
+};
+
 static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int32_t num_q_heads,
                              int64_t q_stride_seq, int64_t q_stride_head, const uint8_t *kv_cache,
                              int64_t num_blocks, int32_t block_size, int64_t stride_block, int64_t stride_token,
@@ -1261,7 +1340,7 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
                              const float *k_centroids, int32_t n_k_centroids, const float *v_centroids,
                              int32_t n_v_centroids, const float *rotation, int32_t rot_block, float sm_scale,
                              void *out, int64_t out_stride_seq, int64_t out_stride_head, void *workspace,
-                             int64_t workspace_bytes, void *stream, KernelEvents ev = {});
+                             int64_t workspace_bytes, void *stream, KernelEvents ev = {}, ShortQueries sq = {});
 
 extern "C" int rq_fused_decode(const void *q, int32_t dtype, int64_t num_seqs, int32_t num_q_heads,
                                int64_t q_stride_seq, int64_t q_stride_head, const uint8_t *kv_cache,
@@ -1377,7 +1456,7 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
                              const float *k_centroids, int32_t n_k_centroids, const float *v_centroids,
                              int32_t n_v_centroids, const float *rotation, int32_t rot_block, float sm_scale,
                              void *out, int64_t out_stride_seq, int64_t out_stride_head, void *workspace,
-                             int64_t workspace_bytes, void *stream, KernelEvents ev) {
+                             int64_t workspace_bytes, void *stream, KernelEvents ev, ShortQueries sq) {
     RQ_CHECK_ARG(dtype == RQ_DTYPE_BF16 || dtype == RQ_DTYPE_F16, "decode dtype must be f16 or bf16");
     RQ_CHECK_ARG(head_dim == kD, "head_dim %d unsupported (only %d)", head_dim, kD);
     RQ_CHECK_ARG(num_kv_heads >= 1 && num_kv_heads <= kMaxKvHeads, "num_kv_heads %d must be 1..%d", num_kv_heads,
@@ -1399,7 +1478,11 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     RQ_CHECK_ARG(((uintptr_t)k_centroids % 16) == 0 && ((uintptr_t)v_centroids % 16) == 0 && ((uintptr_t)rotation % 16) == 0,
                  "centroids and rotation must be 16-byte aligned");
     if (num_seqs == 0) return RQ_OK;
-    RQ_CHECK_SPACE(workspace_bytes >= rq_fused_decode_workspace_bytes(num_seqs, num_q_heads, head_dim, max_seq_len),
+    // Entries of the tile list and columns of the partials: sequences and query heads, or with
+    // short queries column groups and (token, query head) pairs.
+    const int64_t entries = num_seqs * sq.vg;
+    const int64_t columns = (int64_t)num_q_heads * sq.tpg;
+    RQ_CHECK_SPACE(workspace_bytes >= rq_fused_decode_workspace_bytes(entries, (int32_t)columns, head_dim, max_seq_len),
                  "workspace too small");
     RQ_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace % 16) == 0, "workspace must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
@@ -1414,6 +1497,12 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     a.H = num_kv_heads;
     a.G = num_q_heads / num_kv_heads;
     a.HQ = num_q_heads;
+    a.GC = a.G * sq.tpg;
+    a.HC = (int)columns;
+    a.cu_q = sq.cu_q;
+    a.tpg = sq.tpg;
+    a.vg = sq.vg;
+    a.causal = sq.causal;
     a.bt = block_table;
     a.bt_ss = bt_stride_seq;
     a.max_blocks = max_blocks;
@@ -1426,7 +1515,7 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     a.rot_block = rot_block;
     a.score_scale = sm_scale * kLog2e;
     {
-        const DecodeWorkspace W(num_seqs, num_q_heads, std::max<int64_t>(max_seq_len, 1));
+        const DecodeWorkspace W(entries, columns, std::max<int64_t>(max_seq_len, 1));
         uint8_t *base = reinterpret_cast<uint8_t *>(workspace);
         a.part_acc = reinterpret_cast<float *>(base + W.part_acc);
         a.part_ml = reinterpret_cast<float *>(base + W.part_ml);
@@ -1449,6 +1538,9 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     // CU instead (config-1 shape, mean per call: V4/K4 143.8 -> 130.3 us, V4/K3 122.4 ->
     // 115.2; 3-bit V keeps eight heads: 88.5 against 100.9 us at four).
     if (n_v_centroids == 16 && a.hpw == 8) a.hpw = 4;
+    // More than 8 columns of short queries: eight heads' query operands (32 KB) would leave one
+    // workgroup per CU; with four heads (16 KB) three fit.
+    if (sq.cu_q != nullptr && a.GC > 8 && a.hpw == 8) a.hpw = 4;
     // token stride in a stage: 128 bytes per head, unpadded (swizzled) for one or two heads
     // per workgroup in the nibble layout; else the index runs plus a 16-byte skew
     a.tok_stride = (a.hpw <= 2 && !dense3) ? 128 * a.hpw : 2 * SlotLayout(num_kv_heads, head_dim, dense3).ib * a.hpw + 16;
@@ -1464,7 +1556,7 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     // the stages, the descriptor ring, the query slot and the two codebooks (the
     // kernel variant of this hpw and layout places them the same way)
     const size_t lds = (size_t)decode_stages(a.hpw, dense3) * a.stage_bytes +
-                       (size_t)decode_ring(a.hpw, dense3) * sizeof(TileDesc) + (size_t)a.hpw * a.G * 256 + 128;
+                       (size_t)decode_ring(a.hpw, dense3) * sizeof(TileDesc) + (size_t)a.hpw * a.GC * 256 + 128;
     int kb = n_k_centroids == 8 ? 3 : 4, vb = n_v_centroids == 8 ? 3 : 4;
     if (a.max_len > 0) {
         if (dtype == RQ_DTYPE_BF16) launch_decode_bits<RQ_DTYPE_BF16>(a, lds, kb, vb, dense3, st, true, {});
@@ -1474,11 +1566,17 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
         // prep kernel of a 131072-token sequence take ~49 us).
         const int pthreads = 64 * std::max(4, std::min(a.H, kMaxWaves));
         const int ny = std::min(64, std::max(3, (a.max_len + 8 * pthreads - 1) / (8 * pthreads)));
-        const dim3 pgrid((unsigned)num_seqs, (unsigned)(1 + ny)), pblock(pthreads);
+        const dim3 pgrid((unsigned)entries, (unsigned)(1 + ny)), pblock(pthreads);
         // query staging sized by the waves launched (it bounds how many workgroups a CU holds)
         const size_t plds = (size_t)(pthreads / 64) * 16 * kD * sizeof(uint16_t);
-        if (dtype == RQ_DTYPE_BF16) hipLaunchKernelGGL(decode_prep_kernel<RQ_DTYPE_BF16>, pgrid, pblock, plds, st, a);
-        else hipLaunchKernelGGL(decode_prep_kernel<RQ_DTYPE_F16>, pgrid, pblock, plds, st, a);
+        const bool bf = dtype == RQ_DTYPE_BF16;
+        if (sq.cu_q == nullptr) {
+            if (bf) hipLaunchKernelGGL((decode_prep_kernel<RQ_DTYPE_BF16, false>), pgrid, pblock, plds, st, a);
+            else hipLaunchKernelGGL((decode_prep_kernel<RQ_DTYPE_F16, false>), pgrid, pblock, plds, st, a);
+        } else {
+            if (bf) hipLaunchKernelGGL((decode_prep_kernel<RQ_DTYPE_BF16, true>), pgrid, pblock, plds, st, a);
+            else hipLaunchKernelGGL((decode_prep_kernel<RQ_DTYPE_F16, true>), pgrid, pblock, plds, st, a);
+        }
         int rc = check_launch("decode_prep_kernel");
         if (rc) return rc;
         if (dtype == RQ_DTYPE_BF16) launch_decode_bits<RQ_DTYPE_BF16>(a, lds, kb, vb, dense3, st, false, ev);
@@ -1488,26 +1586,97 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     }
     // One wave per (sequence, query head): four per workgroup, or one when the batch has
     // few (sequence, head) pairs, so that they spread over all CUs.
-    const int mw = num_seqs * (int64_t)num_q_heads >= 4LL * device_cus() ? 4 : 1;
+    const int mw = entries * columns >= 4LL * device_cus() ? 4 : 1;
     // Few pairs whose sequences span many decode workgroups each (at least 8 on
     // average: a tensor-parallel slice, a small batch of long contexts): four waves
     // per pair, each taking every fourth segment pass.
-    const bool split = mw == 1 && a.grid_w >= 8 * num_seqs;
-    dim3 mgrid(split ? num_q_heads : (num_q_heads + mw - 1) / mw, (unsigned)num_seqs), mblock(64 * (split ? 4 : mw));
+    const bool split = mw == 1 && a.grid_w >= 8 * entries;
+    dim3 mgrid((unsigned)(split ? columns : (columns + mw - 1) / mw), (unsigned)entries), mblock(64 * (split ? 4 : mw));
     // 32-segment passes when a sequence may span many decode workgroups (very long
     // contexts), or when all merge waves fit at once at the lower occupancy
     // (3 per SIMD); otherwise 16 (config 2: 8192 short merges).  Split merges take
     // 16 while the four waves' first passes cover the average sequence's segments.
-    const bool wide = split ? a.grid_w >= 48 * num_seqs
-                            : a.max_len >= 65536 || num_seqs * (int64_t)num_q_heads <= 12LL * device_cus();
-    auto launch_merge = [&](auto dt) {
+    const bool wide = split ? a.grid_w >= 48 * entries
+                            : a.max_len >= 65536 || entries * columns <= 12LL * device_cus();
+    auto launch_merge = [&](auto dt, auto short_queries) {
         constexpr int DT = decltype(dt)::value;
-        if (split && wide) hipLaunchKernelGGL((decode_merge_kernel<DT, 32, 4>), mgrid, mblock, 0, st, a);
-        else if (split) hipLaunchKernelGGL((decode_merge_kernel<DT, 16, 4>), mgrid, mblock, 0, st, a);
-        else if (wide) hipLaunchKernelGGL((decode_merge_kernel<DT, 32, 1>), mgrid, mblock, 0, st, a);
-        else hipLaunchKernelGGL((decode_merge_kernel<DT, 16, 1>), mgrid, mblock, 0, st, a);
+        constexpr bool S = decltype(short_queries)::value;
+        if (split && wide) hipLaunchKernelGGL((decode_merge_kernel<DT, 32, 4, S>), mgrid, mblock, 0, st, a);
+        else if (split) hipLaunchKernelGGL((decode_merge_kernel<DT, 16, 4, S>), mgrid, mblock, 0, st, a);
+        else if (wide) hipLaunchKernelGGL((decode_merge_kernel<DT, 32, 1, S>), mgrid, mblock, 0, st, a);
+        else hipLaunchKernelGGL((decode_merge_kernel<DT, 16, 1, S>), mgrid, mblock, 0, st, a);
     };
-    if (dtype == RQ_DTYPE_BF16) launch_merge(std::integral_constant<int, RQ_DTYPE_BF16>{});
-    else launch_merge(std::integral_constant<int, RQ_DTYPE_F16>{});
+    auto launch_merge_dt = [&](auto dt) {
+        if (sq.cu_q == nullptr) launch_merge(dt, std::false_type{});
+        else launch_merge(dt, std::true_type{});
+    };
+    if (dtype == RQ_DTYPE_BF16) launch_merge_dt(std::integral_constant<int, RQ_DTYPE_BF16>{});
+    else launch_merge_dt(std::integral_constant<int, RQ_DTYPE_F16>{});
     return check_launch("decode_merge_kernel");
+}
+
+// ---------------------------------------------------------------------------
+// Short queries
+// ---------------------------------------------------------------------------
+
+// What bounds it: as the decode, the table lookups and the stream of keys, once per column group.
+// 32 sequences of 600-8000 keys, 32 / 8 heads, 1 to 8 tokens each (two groups): 87 us, where
+// rq_paged_attention, which unpacks every 64-key tile into LDS and holds one (sequence, kv
+// head) per workgroup, takes 436; its time does not fall with fewer tokens, so four groups
+// are still the better half of it.
+// Columns of a kv head that a column group fills (an MFMA has 16), and the most groups per
+// sequence: every group streams the sequence's keys again (from the caches where they still
+// are there) and looks them up again.
+constexpr int kShortCols = 16, kShortGroups = 4;
+
+static ShortQueries short_shape(int32_t num_q_heads, int32_t num_kv_heads, int64_t max_q_len) {
+    ShortQueries sq;
+    sq.tpg = 0;
+    if (num_kv_heads < 1 || num_q_heads < 1 || num_q_heads % num_kv_heads != 0 || max_q_len < 1) return sq;
+    const int G = num_q_heads / num_kv_heads;
+    if (G > kShortCols) return sq;
+    const int64_t tpg = std::min<int64_t>(kShortCols / G, max_q_len);
+    if ((max_q_len + tpg - 1) / tpg > kShortGroups) return sq;
+    sq.tpg = (int)tpg;
+    sq.vg = (int)((max_q_len + tpg - 1) / tpg);
+    return sq;
+}
+
+extern "C" int64_t rq_short_attention_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                                      int64_t max_q_len, int64_t max_seq_len) {
+    const ShortQueries sq = short_shape(num_q_heads, num_kv_heads, max_q_len);
+    // (entries are a grid's y dimension in the merge, and divided as 32-bit numbers)
+    if (sq.tpg == 0 || num_seqs < 0 || num_seqs * sq.vg > 65535) return 0;
+    return rq_fused_decode_workspace_bytes(num_seqs * sq.vg, num_q_heads * sq.tpg, kD, max_seq_len);
+}
+
+extern "C" int rq_short_attention(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,
+                                  int64_t q_stride_tok, int64_t q_stride_head, const int32_t *cu_seqlens_q,
+                                  int64_t num_seqs, int64_t max_q_len, int32_t causal, const uint8_t *kv_cache,
+                                  int64_t num_blocks, int32_t block_size, int64_t stride_block, int64_t stride_token,
+                                  int32_t num_kv_heads, int32_t head_dim, int32_t index_layout,
+                                  const int32_t *block_table, int64_t max_blocks, int64_t bt_stride_seq,
+                                  const int32_t *seq_lens, int64_t max_seq_len, const float *k_centroids,
+                                  int32_t n_k_centroids, const float *v_centroids, int32_t n_v_centroids,
+                                  const float *rotation, int32_t rot_block, float sm_scale, void *out,
+                                  int64_t out_stride_tok, int64_t out_stride_head, void *workspace,
+                                  int64_t workspace_bytes, void *stream) {
+    RQ_CHECK_ARG(total_q >= 0 && max_q_len >= 0 && num_seqs >= 0, "bad sizes");
+    RQ_CHECK_ARG(num_kv_heads >= 1 && num_q_heads % num_kv_heads == 0, "num_q_heads %d / num_kv_heads %d", num_q_heads,
+                 num_kv_heads);
+    if (num_seqs == 0 || max_q_len == 0 || total_q == 0) return RQ_OK;
+    ShortQueries sq = short_shape(num_q_heads, num_kv_heads, max_q_len);
+    RQ_CHECK_ARG(sq.tpg > 0 && num_seqs * sq.vg <= 65535,
+                 "%lld query tokens of %d heads per kv head take more than %d groups of %d columns, or too many sequences",
+                 (long long)max_q_len, num_q_heads / num_kv_heads, kShortGroups, kShortCols);
+    RQ_CHECK_ARG(cu_seqlens_q != nullptr, "null pointer");
+    RQ_CHECK_ARG(((uintptr_t)out % 4) == 0 && (out_stride_tok * 2) % 4 == 0 && (out_stride_head * 2) % 4 == 0,
+                 "out rows must be 4-byte aligned");
+    sq.cu_q = cu_seqlens_q;
+    sq.causal = causal != 0;
+    return fused_decode_impl(q, dtype, num_seqs, num_q_heads, q_stride_tok, q_stride_head, kv_cache, num_blocks,
+                             block_size, stride_block, stride_token, num_kv_heads, head_dim, index_layout, block_table,
+                             max_blocks, bt_stride_seq, seq_lens, max_seq_len, k_centroids, n_k_centroids,
+                             v_centroids, n_v_centroids, rotation, rot_block, sm_scale, out, out_stride_tok,
+                             out_stride_head, workspace, workspace_bytes, stream, {}, sq);
 }

@@ -56,6 +56,11 @@ _SIGNATURES = {
                                   _c_i64, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_p, _c_i64, _c_i64,
                                   _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i32, _c_p, _c_i32, _c_f32, _c_p, _c_i64, _c_i64,
                                   _c_p, _c_i64, _c_p]),
+    "rq_short_attention_workspace_bytes": (_c_i64, [_c_i64, _c_i32, _c_i32, _c_i64, _c_i64]),
+    "rq_short_attention": (_c_i32, [_c_p, _c_i32, _c_i64, _c_i32, _c_i64, _c_i64, _c_p, _c_i64, _c_i64, _c_i32, _c_p,
+                                    _c_i64, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_p, _c_i64, _c_i64,
+                                    _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i32, _c_p, _c_i32, _c_f32, _c_p, _c_i64, _c_i64,
+                                    _c_p, _c_i64, _c_p]),
 }
 
 EXPORTED = tuple(_SIGNATURES)

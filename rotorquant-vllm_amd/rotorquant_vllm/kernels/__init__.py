@@ -390,6 +390,40 @@ def fused_paged_rq_decode_launcher(q: torch.Tensor, kv_cache: torch.Tensor, bloc
     return launch
 
 
+def _prefill_workspace(dev, workspace, need: int, short_need: int) -> torch.Tensor:
+    """Scratch of a prefill call: the caller's buffer if it holds the tile images (need), else the shared
+    one, large enough for the short-query kernels too when the call can take them."""
+    if workspace is not None and workspace.numel() >= need:
+        return workspace
+    return shared_workspace(dev, "prefill", max(need, short_need))
+
+
+# ---------------------------------------------------------------------------
+# Short queries: attention of a few new tokens per sequence on the decode kernels
+# ---------------------------------------------------------------------------
+
+# Workspace above which a call keeps the kernels that need none or less of it (the
+# partials take 0.5 KB per (token, head) column and workgroup, the descriptors 8.5
+# bytes per key of the block table's capacity and column group).
+_SHORT_WORKSPACE_LIMIT = 256 << 20
+
+
+def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc) -> int:
+    """Workspace of rq_short_attention for this call, or 0 when the call does not take it.
+
+    It is the faster one wherever it takes the call (at most four groups of 16 (token, query head)
+    columns per kv head): 32 sequences of 600-8000 keys, 32 / 8 heads, up to 8 tokens each,
+    437 us in rq_paged_attention, 87 us here."""
+    if not 1 <= max_q_len <= 16 or num_kv_heads > 64 or max_seq_len < 1 or kv_cache.shape[0] < 1:
+        return 0
+    if kc.numel() not in (8, 16) or vc.numel() not in (8, 16) or kc.data_ptr() % 16 or vc.data_ptr() % 16:
+        return 0
+    if kv_cache.data_ptr() % 16 or kv_cache.stride(0) % 16 or kv_cache.stride(1) % 16:
+        return 0
+    need = L.rq_short_attention_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
+    return need if need <= _SHORT_WORKSPACE_LIMIT else 0
+
+
 # ---------------------------------------------------------------------------
 # Fused prefill
 # ---------------------------------------------------------------------------
@@ -456,15 +490,19 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
         max_seq_len = bt.shape[1] * block_size
     L = _lib.load()
     need = L.rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len)
-    ws = workspace if workspace is not None and workspace.numel() >= need else shared_workspace(dev, "prefill", need)
-    rc = L.rq_int8_prefill(
+    short_len = min(max_seq_len, bt.shape[1] * block_size)
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc)
+    ws = _prefill_workspace(dev, workspace, need, sneed)
+    short = sneed and ws.numel() >= sneed
+    fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_int8_prefill, "rq_int8_prefill")
+    rc = fn(
         q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
-        num_seqs, max_q_len, kv_cache.data_ptr(), kv_cache.shape[0], block_size, kv_cache.stride(0),
+        num_seqs, max_q_len, *((1,) if short else ()), kv_cache.data_ptr(), kv_cache.shape[0], block_size, kv_cache.stride(0),
         kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1], bt.stride(0),
-        seq_lens.contiguous().data_ptr(), max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(),
+        seq_lens.contiguous().data_ptr(), short_len if short else max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(),
         R.data_ptr(), blk, float(sm_scale), out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws.numel(),
         _lib.stream_ptr(dev))
-    _lib.check(rc, "rq_int8_prefill")
+    _lib.check(rc, name)
     return out
 
 
@@ -481,7 +519,8 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
 
     The reference's non-fused path (rq_backend.py:937-1036: q_rot = q R^T cast to
     q's dtype, paged decompress to q's dtype, flash_attn_varlen_func, out_rot R)
-    as one kernel that dequantizes K/V tiles into LDS (rq_paged_attention).
+    as one kernel that dequantizes K/V tiles into LDS (rq_paged_attention), or for a few
+    tokens per sequence on the decode kernels (rq_short_attention).
     q: (num_tokens, H_Q, D); cu_seqlens_q (num_seqs + 1,) int32; seq_lens
     (num_seqs,) int32 context lengths including the new tokens; max_q_len: a host
     int bounding every q_len (it sizes the grid).  Query i of sequence b sits at
@@ -507,13 +546,22 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     kc, vc = _f32(k_centroids, dev), _f32(v_centroids, dev)
     cu, sl = cu_seqlens_q.contiguous(), seq_lens.contiguous()
     L = _lib.load()
-    rc = L.rq_paged_attention(
-        q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
-        sl.numel(), int(max_q_len), 1 if causal else 0, kv_cache.data_ptr(), kv_cache.shape[0], block_size,
-        kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1],
-        bt.stride(0),
-        sl.data_ptr(), kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale),
-        out.data_ptr(), out.stride(0), out.stride(1), _lib.stream_ptr(dev))
+    head = (q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
+            sl.numel(), int(max_q_len), 1 if causal else 0, kv_cache.data_ptr(), kv_cache.shape[0], block_size,
+            kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1],
+            bt.stride(0), sl.data_ptr())
+    tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale),
+            out.data_ptr(), out.stride(0), out.stride(1))
+    max_seq_len = bt.shape[1] * block_size
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc)
+    if sneed:
+        # scratch of this call alone, from the stream's allocator: the call stays usable on several
+        # streams at once, as the workspace-free kernel is
+        ws = torch.empty(sneed, dtype=torch.uint8, device=dev)
+        rc = L.rq_short_attention(*head, max_seq_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+        _lib.check(rc, "rq_short_attention")
+        return out
+    rc = L.rq_paged_attention(*head, *tail, _lib.stream_ptr(dev))
     _lib.check(rc, "rq_paged_attention")
     return out
 
@@ -556,13 +604,18 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
         max_seq_len = bt.shape[1] * block_size
     L = _lib.load()
     need = L.rq_paged_prefill_workspace_bytes(sl.numel(), num_kv_heads, max_seq_len)
-    ws = workspace if workspace is not None and workspace.numel() >= need else shared_workspace(dev, "prefill", need)
-    rc = L.rq_paged_prefill(
+    short_len = min(max_seq_len, bt.shape[1] * block_size)
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc)
+    ws = _prefill_workspace(dev, workspace, need, sneed)
+    short = sneed and ws.numel() >= sneed
+    fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_paged_prefill, "rq_paged_prefill")
+    rc = fn(
         q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
         sl.numel(), int(max_q_len), 1 if causal else 0, kv_cache.data_ptr(), kv_cache.shape[0], block_size,
         kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1],
-        bt.stride(0), sl.data_ptr(), max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(),
+        bt.stride(0), sl.data_ptr(), short_len if short else max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(),
+        vc.numel(), R.data_ptr(),
         blk, float(sm_scale), out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws.numel(),
         _lib.stream_ptr(dev))
-    _lib.check(rc, "rq_paged_prefill")
+    _lib.check(rc, name)
     return out

@@ -152,6 +152,46 @@ def test_attention_position_group_edges(H, HQ, mode, dtype, entry):
     check(attn_case(74 + HQ, q_lens, ctx, H, HQ, Params(mode, 4, 3), dtype=dtype), f"groups-{HQ}", entry=entry)
 
 
+@pytest.mark.parametrize("H,HQ,longest,bits,dtype,causal", [
+    (8, 32, 4, (3, 3), torch.bfloat16, True),     # one group of 16 columns
+    (8, 32, 16, (3, 3), torch.bfloat16, True),    # four groups
+    (8, 32, 6, (4, 4), torch.float16, False),
+    (4, 28, 8, (3, 4), torch.bfloat16, True),     # 7 heads: two tokens a group
+    (4, 8, 3, (3, 3), torch.bfloat16, True),      # 6 of 8 columns
+    (2, 24, 4, (4, 3), torch.bfloat16, True),     # 12 heads: one token a group
+    (1, 1, 16, (3, 3), torch.float16, True),      # 16 tokens of one head
+    (3, 48, 2, (3, 3), torch.bfloat16, True),     # 16 heads
+])
+def test_attention_short_queries(H, HQ, longest, bits, dtype, causal, entry):
+    """Queries of 1 to 16 tokens (the decode kernels' column groups): contexts at the 32-key tile's edges, at
+    the query's own length (the first token sees one key), ending a token into a tile (which the
+    query's first tokens do not see), and long enough for several workgroups; sequences without tokens."""
+    q_lens = [longest, 1, 0, max(1, longest - 1), longest, min(2, longest), longest, 0]
+    ctx = [longest, 1, 40, 33, 64, 31 + min(2, longest), 3000, 0]
+    check(attn_case(90 + HQ, q_lens, ctx, H, HQ, Params("iso" if H != 3 else "planar", *bits), dtype=dtype),
+          f"short-{HQ}-{longest}", causal=causal, entry=entry)
+
+
+def test_attention_short_queries_more_than_keys():
+    """More query tokens than keys: the tokens before the first key see none and give zeros; and the fused
+    prefill's call of the same batch, with the caller's scratch too small for the short-query kernels."""
+    from rotorquant_vllm import kernels as K
+    case = attn_case(89, [5, 3], [2, 40], 2, 8, Params("iso", 3, 3))
+    p = case["p"]
+    got = run(case)
+    assert np.isfinite(got).all() and (got[:3] == 0).all() and (got[3:] != 0).any(axis=(1, 2)).all()
+    args = (_dev(case["q"]), _dev(case["cache"]), _dev(case["bt"]), _dev(case["lens"]), _dev(p.kc), _dev(p.vc), _dev(p.R), 2, 128, 16)
+    small = torch.empty(2 * 2 * 33792, dtype=torch.uint8, device="cuda")
+    for ws in (None, small):
+        out = torch.zeros_like(args[0])
+        K.fused_paged_rq_int8_prefill(*args, out=out, cu_seqlens_q=_dev(case["cu"]), max_q_len=5, max_seq_len=40, workspace=ws)
+        torch.cuda.synchronize()
+        o = out.float().cpu().numpy()
+        assert (o[:3] == 0).all()
+        err, excess, cs = check_tolerance(o[3:], got[3:], "bfloat16", rot_block=p.blk)
+        assert excess <= 0 and cs >= 0.999, (err, excess, cs)
+
+
 def test_attention_graph_replay():
     """The call captured in a HIP graph: each replay, after the eager work between
     replays (new q and context lengths written into the captured buffers), equals
