@@ -151,6 +151,14 @@ def test_decode_k3_v4_and_block_size_32():
     check(decode_case(5, 3, 8, 16, lens, block_size=32, p=p), "k3v4-bs32")
 
 
+@pytest.mark.parametrize("bits,tiles", [(3, 511), (3, 512), (3, 513), (4, 383), (4, 385), (3, 1)])
+def test_decode_tiles_around_the_workgroup_count(bits, tiles):
+    """As many 32-key tiles as decode workgroups (two per CU with 3-bit codebooks, one and a half with
+    4-bit ones), one fewer and one more: one tile per workgroup, or ranges by weight."""
+    case = decode_case(16, 2, 8, 32, [32 * (tiles - 1), 5] if tiles > 1 else [5, 0], p=Params("iso", bits, bits))
+    check(case, f"tiles-{bits}-{tiles}")
+
+
 def test_decode_closed_forms():
     """Closed forms, no attention oracle: L = 1 -> the R-rotated V row; identical keys
     (every cached key the same vector) -> the R-rotated mean of V, at 8 kv heads x GQA 4
