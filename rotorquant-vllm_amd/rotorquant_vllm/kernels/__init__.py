@@ -48,11 +48,12 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "rotorquant_vllm.kernels runs only on ROCm device tensors (got a "
                 f"{t.device.type} tensor); there is no CPU path")
-        dev = t.device if dev is None else dev
+        if dev is None:
+            dev = t.device
     _lib.load()
     return dev
 
@@ -116,7 +117,14 @@ def _rt_block(rot_T_even: torch.Tensor, rot_T_odd: torch.Tensor) -> int:
 
 
 def _f32(t: torch.Tensor, device) -> torch.Tensor:
+    # (a launch of a few microseconds waits for these checks; .to() and .contiguous() cost three times as much)
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.float32).contiguous()
+
+
+def _i32(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype is torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
 
 
 def _layout(dense3: bool) -> int:
@@ -211,7 +219,9 @@ def compress_store(key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tenso
     if kv_cache.dtype != torch.uint8 or kv_cache.dim() != 3:
         raise ValueError("kv_cache must be a (num_blocks, block_size, total_bytes) uint8 tensor")
     blk = rot_block if rot_block is not None else _rt_block(rot_T_even, rot_T_odd)
-    sm = slot_mapping.to(torch.int64).contiguous()
+    sm = slot_mapping
+    if sm.dtype is not torch.int64 or not sm.is_contiguous():
+        sm = sm.to(torch.int64).contiguous()
     if sm.numel() < N:
         raise ValueError("slot_mapping shorter than the number of tokens")
     N = min(N, sm.numel())
@@ -248,7 +258,7 @@ def paged_decompress(kv_cache: torch.Tensor, block_table: torch.Tensor, seq_lens
     bt = block_table.to(torch.int32)
     if bt.stride(-1) != 1:
         bt = bt.contiguous()
-    sl = seq_lens.to(torch.int32).contiguous()
+    sl = _i32(seq_lens)
     B, MB = bt.shape
     cap = NB if out_k is None else out_k.shape[0]
     if out_k is None:
@@ -485,7 +495,7 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
     blk = rotation_block(rotation)
     R = _f32(rotation, dev)
     kc, vc = _f32(k_centroids, dev), _f32(v_centroids, dev)
-    cu = cu_seqlens_q.to(torch.int32).contiguous()
+    cu = _i32(cu_seqlens_q)
     if max_seq_len is None:
         max_seq_len = bt.shape[1] * block_size
     L = _lib.load()
