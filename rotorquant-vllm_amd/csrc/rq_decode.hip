@@ -350,12 +350,18 @@ __device__ __forceinline__ void wait_copies_upto(int n) {
 // Tile descriptor: one 32-token tile of one sequence, written by the prep kernel
 // and read by the decode workgroup that owns the tile.
 struct TileDesc {
-    int32_t seq, tile, valid;       // entry, tile index inside it, tokens in the tile (1..32)
-    int32_t lim;                    // tokens of the tile that the entry's first query token sees (each
-                                    // following token one more, up to valid); valid when all see the tile
+    int32_t seq, tile;  // entry, tile index inside it
+    int32_t vl;         // pack_vl(valid, lim) (valid alone without short queries): valid = tokens in the tile (1..32); lim = those of them that the
+                        // entry's first query token sees (each following token one more, up to valid)
+    int32_t pad;
     uint64_t off[kTile];            // byte offset of each token's slot (0 past `valid`)
 };
 static_assert(sizeof(TileDesc) == 16 + 8 * kTile, "TileDesc layout");
+template <bool SHORT>
+__device__ __forceinline__ int pack_vl(int valid, int lim) { return SHORT ? valid | (max(lim, -64) + 64) << 8 : valid; }
+template <bool SHORT>
+__device__ __forceinline__ int vl_valid(int vl) { return SHORT ? vl & 0xff : vl; }
+__device__ __forceinline__ int vl_lim(int vl) { return (vl >> 8) - 64; }
 constexpr int kDescPieces = (int)sizeof(TileDesc) / 16;  // 16-byte copy pieces per descriptor
 
 // Pipeline depth of a decode variant (hpw kv heads per workgroup, dense layout d3):
@@ -384,9 +390,7 @@ static_assert(decode_ring(1, false) >= 2 * decode_stages(1, false) && decode_rin
 // The split is s(w) * M >> 32 with M ~ NT 2^32 / s(grid_w) (M = the high half of
 // (NT << 32) * split_r, at most the exact quotient), computed once by the prep
 // kernel; the decode and the merge kernel evaluate exactly this, and the last
-// range ends at NT.  With no more tiles than workgroups, workgroup w takes tile w: spread over
-// all of them by weight, the few tiles' partials lay among hundreds of empty ranges that the
-// merge had to pass over (one sequence of 777 keys, 25 tiles: merge 10.9 -> 5.7 us, call 22.5 -> 18.6).
+// range ends at NT.
 struct RangeSplit {
     int c, G, NT;
     int w0, w1, w2, w3;  // rank weights
@@ -396,13 +400,16 @@ __device__ __forceinline__ uint64_t split_multiplier(const DecodeArgs &a, int NT
     return __umul64hi((uint64_t)NT << 32, a.split_r);
 }
 __device__ __forceinline__ RangeSplit make_split(const DecodeArgs &a, int NT) {
-    return RangeSplit{a.split_c, a.grid_w, NT, a.wt[0], a.wt[1], a.wt[2], a.wt[3], *a.split_m};
+    // (loaded here, with the tile count: sunk into the branch on that count the two loads would
+    // follow one another, 0.5 us at the start of every decode workgroup)
+    uint64_t M = *a.split_m;
+    asm volatile("" : "+s"(M));
+    return RangeSplit{a.split_c, a.grid_w, NT, a.wt[0], a.wt[1], a.wt[2], a.wt[3], M};
 }
 // r by value: through a reference the rank select below is turned into an indexed
 // load of the struct, which the compiler then moves to LDS.
-__device__ __forceinline__ int range_start(const RangeSplit r, int w) {
+__device__ __forceinline__ int weighted_start(const RangeSplit r, int w) {
     if (w >= r.G) return r.NT;
-    if (r.NT <= r.G) return min(w, r.NT);
     const int rank = min(w / r.c, 3);
     const int wr = rank == 0 ? r.w0 : rank == 1 ? r.w1 : rank == 2 ? r.w2 : r.w3;
     uint64_t s = (uint64_t)(w - rank * r.c) * wr;
@@ -412,6 +419,13 @@ __device__ __forceinline__ int range_start(const RangeSplit r, int w) {
     return (int)((s * r.M) >> 32);
 }
 
+// With no more tiles than workgroups, workgroup w takes tile w: spread over all of them by
+// weight, the few tiles' partials lay among hundreds of empty ranges that the merge had to pass
+// over (one sequence of 777 keys, 25 tiles: merge 10.9 -> 5.7 us, call 22.5 -> 18.6).
+__device__ __forceinline__ bool tile_per_workgroup(const RangeSplit &r) { return r.NT <= r.G; }
+__device__ __forceinline__ int range_start(const RangeSplit r, int w) {
+    return tile_per_workgroup(r) ? min(w, r.NT) : weighted_start(r, w);
+}
 
 template <bool SHORT>
 __device__ __forceinline__ int seq_tiles(const DecodeArgs &a, int64_t e) {
@@ -487,14 +501,15 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
         // + k within the bracket (step <= 64 while G <= 4097; beyond that a lane loop).
         const int step = (r.G - 1 + 63) / 64;
         auto count_le = [&](int tk) {
+            if (tile_per_workgroup(r)) return max(tk, 0);
             const int w1 = 1 + lane * step;
-            const uint64_t m1 = __ballot(w1 < r.G && range_start(r, w1) <= tk);
+            const uint64_t m1 = __ballot(w1 < r.G && weighted_start(r, w1) <= tk);
             const int k = m1 ? 63 - __clzll(m1) : -1;  // last coarse point at or below tk
             if (k < 0) return 0;
             int c = k * step + 1;  // w = 1 .. 1 + k * step all count
             for (int j0 = 1; j0 < step; j0 += 64) {
                 const int w2 = 1 + k * step + j0 + lane;
-                const uint64_t m2 = __ballot(j0 + lane < step && w2 < r.G && range_start(r, w2) <= tk);
+                const uint64_t m2 = __ballot(j0 + lane < step && w2 < r.G && weighted_start(r, w2) <= tk);
                 c += __popcll(m2);
             }
             return c;
@@ -537,8 +552,8 @@ __global__ __launch_bounds__(512) void decode_prep_kernel(DecodeArgs a) {
         if (j0 % kTile == 0) {
             d->seq = (int32_t)seq;
             d->tile = j0 / kTile;
-            d->valid = min(kTile, L - j0);
-            d->lim = min(kTile, L0 - j0);
+            d->vl = pack_vl<SHORT>(min(kTile, L - j0), min(kTile, L0 - j0));
+            d->pad = 0;
         }
     }
 }
@@ -574,8 +589,10 @@ constexpr int decode_waves_per_eu(int kb, int vb, int hpw) {
 }
 
 // D3: the cache holds the dense 3-bit index layout (48 index bytes per head).
-// WIDE: more than 8 query heads per kv head.
-template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE>
+// WIDE: more than 8 columns (query heads, or with SHORT (token, query head) pairs) per kv head.
+// SHORT: entries of several query tokens, whose causal limits differ by column (as a run-time choice it cost
+// the two-head variant 2 %).
+template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE, bool SHORT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_waves_per_eu(KB, VB, HPW)))) void decode_kernel(DecodeArgs a) {
     const int w = blockIdx.x;
     const int NT = *a.n_tiles_total;
@@ -632,7 +649,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
     // token copies (line copies: four) and one norm copy (HPW >= 4: on waves < hpw / 4).
     auto issue = [&](int i, const uint8_t *sb) {
         const TileDesc &d = ring[i & (RING - 1)];
-        const int valid = __builtin_amdgcn_readfirstlane(d.valid);
+        const int valid = vl_valid<SHORT>(__builtin_amdgcn_readfirstlane(d.vl));
         int n = 0;
         const uint64_t base = d.off[lane_now() & 31];
         const uint32_t dst = lds_addr(sb);
@@ -814,8 +831,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         __syncthreads();
 
         const int tseq = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].seq);
-        const int valid = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].valid);
-        const int qlim = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].lim);
+        const int vl = __builtin_amdgcn_readfirstlane(ring[t & (RING - 1)].vl);
+        const int valid = vl_valid<SHORT>(vl);
+        const int qlim = SHORT ? vl_lim(vl) : valid;
         if (tseq != seq) {  // a new sequence starts at this tile
             if (seq >= 0) end_segment();
             seq = tseq;
@@ -986,10 +1004,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         // commutes with).
         float s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
         if (qlim < kTile) {
-            // (this lane's query token of the entry: its column / G)
+            // (this lane's query token of the entry is its column / G)
             const uint32_t ln = lane_now();
-            const int tok = (int)((WIDE ? ln & 15u : ln & 7u) / (uint32_t)opaque_s(a.G));
-            const int vv = min(valid, opaque_s(qlim) + tok);
+            int vv = opaque_s(qlim);
+            if constexpr (SHORT) vv = min(valid, vv + (int)((WIDE ? ln & 15u : ln & 7u) / (uint32_t)opaque_s(a.G)));
             const int g4 = 4 * (int)(ln >> 4);
     #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -1110,7 +1128,10 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     const int n = seq_tiles<SHORT>(a, seq);
     const int w_lo = n > 0 ? tp_lo : 0, nch = n > 0 ? tp_n : 0;
     const RangeSplit rsp = make_split(a, ntt);
-    auto has_tiles = [rsp](int w) { return range_start(rsp, w + 1) > range_start(rsp, w); };
+    const bool all_have_tiles = tile_per_workgroup(rsp);
+    auto has_tiles = [rsp, all_have_tiles](int w) {
+        return all_have_tiles || weighted_start(rsp, w + 1) > weighted_start(rsp, w);
+    };
     const float *ml = a.part_ml + (w_lo + seq) * (int64_t)(SHORT ? a.HC : a.HQ) * 2 + hq * 2;
     const float *pa = a.part_acc + (w_lo + seq) * (int64_t)(SHORT ? a.HC : a.HQ) * kD + hq * kD;
     const int64_t cs_ml = (int64_t)(SHORT ? a.HC : a.HQ) * 2, cs_acc = (int64_t)(SHORT ? a.HC : a.HQ) * kD;
@@ -1206,7 +1227,7 @@ constexpr int decode_slot_factor(int64_t num_q_heads) { return num_q_heads <= 16
 // Resident decode workgroups per CU for an LDS size (cached per device and size;
 // the cache of each kernel instance is guarded by a mutex, so concurrent callers
 // see whole entries).
-template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE>
+template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE, bool SHORT>
 static int decode_per_cu(const DecodeArgs &a, size_t lds) {
     static int cache[64][8][2] = {};  // [device][entry] = {lds, workgroups per CU}
     static std::mutex mu;
@@ -1220,7 +1241,7 @@ static int decode_per_cu(const DecodeArgs &a, size_t lds) {
     }
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &nb, reinterpret_cast<const void *>(&decode_kernel<DT, KB, VB, HPW, D3, WIDE>), 64 * a.hpw, lds) !=
+            &nb, reinterpret_cast<const void *>(&decode_kernel<DT, KB, VB, HPW, D3, WIDE, SHORT>), 64 * a.hpw, lds) !=
             hipSuccess ||
         nb <= 0)
         nb = 1;
@@ -1244,19 +1265,19 @@ struct KernelEvents {
 
 // configure: set the grid and range split only (before the prep kernel, which
 // needs them); otherwise launch.
-template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE>
+template <int DT, int KB, int VB, int HPW, bool D3, bool WIDE, bool SHORT>
 static void launch_decode_h(DecodeArgs &a, size_t lds, hipStream_t st, bool configure, KernelEvents ev) {
     if (!configure) {
         const dim3 grid((unsigned)a.grid_w, 1, a.H / a.hpw), block(64 * a.hpw);
         if (ev.start != nullptr || ev.stop != nullptr)  // events at this kernel's own start and end
-            hipExtLaunchKernelGGL((decode_kernel<DT, KB, VB, HPW, D3, WIDE>), grid, block, lds, st, ev.start, ev.stop, 0,
+            hipExtLaunchKernelGGL((decode_kernel<DT, KB, VB, HPW, D3, WIDE, SHORT>), grid, block, lds, st, ev.start, ev.stop, 0,
                                   a);
         else
-            hipLaunchKernelGGL((decode_kernel<DT, KB, VB, HPW, D3, WIDE>), grid, block, lds, st, a);
+            hipLaunchKernelGGL((decode_kernel<DT, KB, VB, HPW, D3, WIDE, SHORT>), grid, block, lds, st, a);
         return;
     }
     // as many workgroups per kv-head group as are resident at once
-    const int per_cu = decode_per_cu<DT, KB, VB, HPW, D3, WIDE>(a, lds);
+    const int per_cu = decode_per_cu<DT, KB, VB, HPW, D3, WIDE, SHORT>(a, lds);
     const int groups = a.H / a.hpw;
     a.grid_w = std::max(1, per_cu * device_cus() / groups);
     // rank weights by workgroups per CU (workgroups [r CUs, (r+1) CUs) are
@@ -1276,19 +1297,24 @@ static void launch_decode_h(DecodeArgs &a, size_t lds, hipStream_t st, bool conf
     a.split_r = UINT64_MAX / tot;
 }
 
-template <int DT, int KB, int VB, bool D3, bool WIDE>
+template <int DT, int KB, int VB, bool D3, bool WIDE, bool SHORT>
 static void launch_decode_w(DecodeArgs &a, size_t lds, hipStream_t st, bool configure, KernelEvents ev) {
-    if (a.hpw == 8) launch_decode_h<DT, KB, VB, 8, D3, WIDE>(a, lds, st, configure, ev);
-    else if (a.hpw == 4) launch_decode_h<DT, KB, VB, 4, D3, WIDE>(a, lds, st, configure, ev);
-    else if (a.hpw == 2) launch_decode_h<DT, KB, VB, 2, D3, WIDE>(a, lds, st, configure, ev);
-    else if (a.hpw == 1) launch_decode_h<DT, KB, VB, 1, D3, WIDE>(a, lds, st, configure, ev);
-    else launch_decode_h<DT, KB, VB, 0, D3, WIDE>(a, lds, st, configure, ev);
+    if constexpr (!(SHORT && WIDE)) {  // (short queries of more than 8 columns take at most four heads)
+        if (a.hpw == 8) return launch_decode_h<DT, KB, VB, 8, D3, WIDE, SHORT>(a, lds, st, configure, ev);
+    }
+    if (a.hpw == 4) launch_decode_h<DT, KB, VB, 4, D3, WIDE, SHORT>(a, lds, st, configure, ev);
+    else if (a.hpw == 2) launch_decode_h<DT, KB, VB, 2, D3, WIDE, SHORT>(a, lds, st, configure, ev);
+    else if (a.hpw == 1) launch_decode_h<DT, KB, VB, 1, D3, WIDE, SHORT>(a, lds, st, configure, ev);
+    else launch_decode_h<DT, KB, VB, 0, D3, WIDE, SHORT>(a, lds, st, configure, ev);
 }
 
 template <int DT, int KB, int VB, bool D3 = false>
 static void launch_decode(DecodeArgs &a, size_t lds, hipStream_t st, bool configure, KernelEvents ev) {
-    if (a.GC > 8) launch_decode_w<DT, KB, VB, D3, true>(a, lds, st, configure, ev);
-    else launch_decode_w<DT, KB, VB, D3, false>(a, lds, st, configure, ev);
+    const bool wide = a.GC > 8, sq = a.cu_q != nullptr;
+    if (wide && sq) launch_decode_w<DT, KB, VB, D3, true, true>(a, lds, st, configure, ev);
+    else if (wide) launch_decode_w<DT, KB, VB, D3, true, false>(a, lds, st, configure, ev);
+    else if (sq) launch_decode_w<DT, KB, VB, D3, false, true>(a, lds, st, configure, ev);
+    else launch_decode_w<DT, KB, VB, D3, false, false>(a, lds, st, configure, ev);
 }
 
 template <int DT>
