@@ -376,6 +376,16 @@ int rq_paged_prefill(const void *q, int32_t dtype, int64_t total_q, int32_t num_
 int64_t rq_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads, int64_t max_seq_len);
 
 /*
+ * Workspace with which rq_int8_prefill / rq_paged_prefill also spread a call of few query
+ * blocks over the whole GPU: the tile images, and fp32 partials of the key chunks that
+ * several workgroups then take of one query block (at most 35 MB more; the same bytes as
+ * rq_int8_prefill_workspace_bytes for calls that fill the GPU by themselves).  With a
+ * workspace between the two sizes, the calls run unsplit.
+ */
+int64_t rq_prefill_split_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                         int64_t max_q_len, int64_t max_seq_len);
+
+/*
  * rq_paged_prefill for queries of a few tokens (drafts being verified), on the
  * kernels of rq_fused_decode: the (token, query head) pairs of a kv head share its
  * stream of packed keys, up to 16 pairs at a time, so nothing is unpacked to memory

@@ -73,6 +73,8 @@ struct PrefillArgs {
     int causal;         // 0: every query sees all seq_lens[b] keys
     int64_t max_tiles;  // tile images per (sequence, kv head) in the workspace
     uint8_t *ws;        // tile images [num_seqs][H][max_tiles][kImBytes]
+    int nx, split;      // query blocks; workgroups per query block (key chunks), > 1: partials in `part`
+    float *part;        // [(seq, kv head, query block, chunk)][wave] partials of kPartFloats
     void *out;
     int64_t o_st, o_sh;
 };
@@ -214,6 +216,36 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(PrefillArgs a) {
     }
 }
 
+// ---- key chunks ---------------------------------------------------------------
+// With few query blocks (a short chunk behind a long prefix) `split` workgroups take the tiles
+// of one query block, each a contiguous run of them, and prefill_merge_kernel adds up their
+// partials: per position the accumulators, and (max in base 2 plus V exponent, row sum).
+// What bounds a call without them: one chain of tiles per query block on a few of the CUs.  One
+// sequence, 32 / 8 heads, whole call: 64 tokens behind 16000 keys 370 -> 70 us; 200 behind 2000
+// 73 -> 38; one 1500-token prompt (which already fills the GPU) 61 -> 47 by the wider waves alone.
+constexpr int kPartFloats = kPW * kPD + kPW * 2;
+constexpr int kMinChunk = 4;  // tiles of a chunk, at least (a workgroup's fixed work is worth about 6)
+__device__ __forceinline__ int chunk_tiles(const PrefillArgs &a, int n_tiles) {
+    return max(kMinChunk, (n_tiles + a.split - 1) / a.split);
+}
+// Query block -> its first unit, unit count of the sequence and key tiles (see prefill_attn_kernel).
+struct QueryBlock {
+    int q0, T, L, units, f0, kv_end, n_tiles;
+};
+__device__ __forceinline__ QueryBlock query_block(const PrefillArgs &a, int64_t seq, int qblk) {
+    QueryBlock b;
+    b.q0 = a.cu_q[seq];
+    b.T = a.cu_q[seq + 1] - b.q0;
+    b.L = a.seq_lens[seq];
+    const int L_eff = visible_keys(a, seq);
+    b.units = b.T > 0 ? (b.T + kPW - 1) / kPW * a.G : 0;
+    b.f0 = qblk * kWaves;
+    const int last_i = min(b.T, (min(b.f0 + kWaves, b.units) - 1) / a.G * kPW + kPW) - 1;
+    b.kv_end = a.causal ? min(L_eff, b.L - b.T + last_i + 1) : L_eff;  // keys [0, kv_end) may be visible
+    b.n_tiles = b.kv_end > 0 ? (b.kv_end + kKT - 1) / kKT : 0;
+    return b;
+}
+
 // ---- attention ----------------------------------------------------------------
 // What bounds it: vector issue and the matrix cores side by side.  A wave's tile is 32 MFMAs of
 // 32 cycles and about 115 vector instructions of 4 with 32 exponentials of 8 to 9; the MFMA unit
@@ -229,27 +261,39 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     int qblk, h;
     int64_t seq;
     attn_work_item(qblk, h, seq);
-    const int q0 = a.cu_q[seq], q1 = a.cu_q[seq + 1];
-    const int T = q1 - q0;
-    const int L = a.seq_lens[seq];
-    const int pos_base = L - T;  // position of query 0
-    const int L_eff = visible_keys(a, seq);
+    int chunk = 0;
+    if (a.split > 1) {
+        chunk = qblk % a.split;
+        qblk /= a.split;
+    }
+    const QueryBlock qb = query_block(a, seq, qblk);
+    const int q0 = qb.q0, T = qb.T, units = qb.units, f0 = qb.f0, kv_end = qb.kv_end;
+    const int pos_base = qb.L - T;  // position of query 0
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int hh = lane >> 5, col = lane & 31;
     // This wave's unit: (32-position group, query head of the GQA group) of the sequence and
     // kv head, in position-group-major order; the workgroup's units span two position
     // groups at most when G >= 4 (whatever G, the four SIMDs carry one wave each).
-    const int units = T > 0 ? (T + kPW - 1) / kPW * a.G : 0;
-    const int f0 = qblk * kWaves;
     if (f0 >= units) return;
     const int f = f0 + wave;
     const int i0 = f < units ? f / a.G * kPW : T;  // first query index (units past the end: inactive)
-    const int last_i = min(T, (min(f0 + kWaves, units) - 1) / a.G * kPW + kPW) - 1;
     const int hq = h * a.G + f % a.G;
     const bool wave_active = i0 < T;
     const int my_i = i0 + col;              // query index of this lane's column
     const int my_pos = pos_base + my_i;
+    // This workgroup's tiles [t0, t0 + n_tiles) and, of those, the first nw that this wave takes part
+    // in (the causal bound of its positions); t below counts from t0.
+    const bool causal = a.causal;
+    int t0 = 0, n_tiles = qb.n_tiles;
+    if (a.split > 1) {
+        const int per = chunk_tiles(a, n_tiles);
+        t0 = chunk * per;
+        n_tiles = min(per, n_tiles - t0);
+        if (n_tiles <= 0) return;  // (the merge does not look at this chunk)
+    }
+    const int wv_end = causal ? min(kv_end, pos_base + i0 + kPW) : kv_end;
+    const int nw = wave_active ? max(0, min(n_tiles, (max(wv_end, 0) + kKT - 1) / kKT - t0)) : 0;
 
     // LDS: two K buffers (K rows and the tile's V exponent) and two V'^T buffers.
     extern __shared__ __align__(16) uint8_t lds[];
@@ -257,16 +301,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     uint8_t *const vbuf[2] = {lds + 2 * kLdsK, lds + 2 * kLdsK + kLdsV};
     float4 *const rot = reinterpret_cast<float4 *>(lds + 2 * (kLdsK + kLdsV));
 
-    // ---- key range: causal bound of the whole workgroup and of this wave -----------
-    const bool causal = a.causal;
-    const int kv_end = causal ? min(L_eff, pos_base + last_i + 1) : L_eff;  // keys [0, kv_end) may be visible
-    const int n_tiles = kv_end > 0 ? (kv_end + kKT - 1) / kKT : 0;
-    const int wv_end = causal ? min(kv_end, pos_base + i0 + kPW) : kv_end;
-    const int nw = wave_active && wv_end > 0 ? (wv_end + kKT - 1) / kKT : 0;  // tiles this wave takes part in
-
     // Tile images of this (sequence, kv head), copied global -> LDS 1 KB per wave instruction.
     // The rotation of the query operand overlaps the first copies.
-    const uint8_t *img0 = a.ws + ((int64_t)seq * a.H + h) * a.max_tiles * kImBytes;
+    const uint8_t *img0 = a.ws + (((int64_t)seq * a.H + h) * a.max_tiles + t0) * kImBytes;
     const uint32_t lds0 = lds_addr(lds);
     auto copy_rows = [&](int t, int from, uint32_t dst_) {
         const uint64_t s = reinterpret_cast<uint64_t>(img0 + (int64_t)t * kImBytes + from);
@@ -314,7 +351,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     int e_v = 0;          // its V exponent
     // Mask of tile t's scores: at the diagonal and the end.
     auto mask = [&](int t, f32x16 (&s)[2]) {
-        const int k0 = t * kKT, nk = min(kKT, kv_end - k0);
+        const int k0 = (t0 + t) * kKT, nk = min(kKT, kv_end - k0);
         // every key of the tile visible to all 32 positions of this wave: no mask
         if (!(nk == kKT && (!causal || k0 + kKT - 1 <= pos_base + i0)))
             wide_mask(s, (causal ? min(k0 + nk, my_pos + 1) : k0 + nk) - (k0 + 4 * hh));
@@ -420,10 +457,72 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     for (; t < n_tiles; ++t) turn(t);  // tiles above this wave's diagonal: only their copies and barriers
     if (!wave_active) return;
 
+    if (a.split > 1) {
+        float *pt = a.part + ((((seq * a.H + h) * a.nx + qblk) * a.split + chunk) * kWaves + wave) * (int64_t)kPartFloats;
+        auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(st.l_run), __float_as_uint(st.l_run), false, false);
+        const float l = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        if (hh == 0)  // m_run = -inf (no key of the chunk seen) stays -inf
+            *reinterpret_cast<float2 *>(pt + kPW * kPD + 2 * col) = make_float2(st.m_run * scale + (float)st.e_run, l);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *reinterpret_cast<float4 *>(pt + col * kPD + 32 * m + 8 * j + 4 * hh) =
+                    make_float4(st.acc[m][4 * j], st.acc[m][4 * j + 1], st.acc[m][4 * j + 2], st.acc[m][4 * j + 3]);
+        return;
+    }
     // ---- epilogue: normalise, round to the q dtype, rotate back by R, round ----
     const bool ovalid = my_i < T;
     uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + (ovalid ? my_i : 0)) * a.o_st + (int64_t)hq * a.o_sh;
     wide_store<DT>(st, ovalid, orow, rot, a.rot_block, hh);
+}
+
+// One workgroup per unit of a split call: thread (position p = tid / 8, part = tid % 8) adds up 16 dims
+// of the chunks' partials, relative to the largest maximum, then the epilogue as above.
+template <int DT>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+    const int f = blockIdx.x, h = blockIdx.y;
+    const int64_t seq = blockIdx.z;
+    const int qblk = f / kWaves;
+    const QueryBlock qb = query_block(a, seq, qblk);
+    if (f >= qb.units) return;
+    __shared__ float4 rot[kPD];
+    load_rotation(rot, a.R, threadIdx.x);
+    __syncthreads();
+    const int p = threadIdx.x >> 3, part = threadIdx.x & 7;
+    const int qi = f / a.G * kPW + p;
+    if (qi >= qb.T) return;
+    const int per = chunk_tiles(a, qb.n_tiles), nch = (qb.n_tiles + per - 1) / per;
+    const int64_t stride = (int64_t)kWaves * kPartFloats;  // between chunks
+    const float *pt = a.part + ((((seq * a.H + h) * a.nx + qblk) * a.split) * kWaves + f % kWaves) * (int64_t)kPartFloats;
+    float M = -INFINITY, l = 0.f, acc[16] = {};
+    for (int c = 0; c < nch; ++c) {
+        const float *pc = pt + c * stride;
+        const float2 ml = *reinterpret_cast<const float2 *>(pc + kPW * kPD + 2 * p);
+        float4 x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const float4 *>(pc + p * kPD + 16 * part + 4 * k);
+        const float Mn = fmaxf(M, ml.x);
+        const float keep = M == Mn ? 1.f : __builtin_amdgcn_exp2f(M - Mn);          // M = -inf: 0
+        const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - Mn);
+        M = Mn;
+        l = l * keep + w * ml.y;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float xs[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[4 * k + i] = acc[4 * k + i] * keep + w * xs[i];
+        }
+    }
+    const float inv_l = l > 0.f ? 1.f / l : 0.f;
+    uint16_t *orow = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(qb.q0 + qi) * a.o_st + (int64_t)(h * a.G + f % a.G) * a.o_sh;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int d0 = 16 * part + 4 * k;
+        const float o[4] = {acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]};
+        *reinterpret_cast<uint2 *>(orow + d0) =
+            a.rot_block == 4 ? rotate_back4<DT, 4>(o, inv_l, d0, rot) : rotate_back4<DT, 2>(o, inv_l, d0, rot);
+    }
 }
 
 template <int DT>
@@ -433,14 +532,35 @@ static void launch_pack(const PrefillArgs &a, int64_t num_seqs, hipStream_t st) 
 }
 
 template <int DT>
-static void launch_attn(const PrefillArgs &a, int64_t num_seqs, int64_t max_q_len, hipStream_t st) {
+static void launch_attn(const PrefillArgs &a, int64_t num_seqs, hipStream_t st) {
     const size_t lds = 2 * (size_t)(kLdsK + kLdsV) + kRotBytes;
-    const int64_t nx = ((max_q_len + kPW - 1) / kPW * a.G + kWaves - 1) / kWaves;
-    dim3 grid((unsigned)nx, (unsigned)a.H, (unsigned)num_seqs);
+    dim3 grid((unsigned)(a.nx * a.split), (unsigned)a.H, (unsigned)num_seqs);
     hipLaunchKernelGGL((prefill_attn_kernel<DT>), grid, dim3(64 * kWaves), lds, st, a);
+    if (a.split > 1) {
+        dim3 mgrid((unsigned)(a.nx * kWaves), (unsigned)a.H, (unsigned)num_seqs);
+        hipLaunchKernelGGL((prefill_merge_kernel<DT>), mgrid, dim3(256), 0, st, a);
+    }
 }
 
 static int64_t prefill_tiles(int64_t max_seq_len) { return (max_seq_len + kKT - 1) / kKT; }
+
+// Query blocks of the longest query, and the key chunks of each: as many as fit the GPU's two
+// workgroups per CU, when that is at least two, of kSplitTiles tiles each by the call's bound on the
+// lengths (the kernel divides each block's own tiles).
+struct PrefillShape {
+    int64_t nx, split;
+};
+constexpr int kSplitTiles = 8;
+static PrefillShape prefill_shape(int64_t num_seqs, int G, int H, int64_t max_q_len, int64_t max_seq_len) {
+    const int64_t nx = ((max_q_len + kPW - 1) / kPW * G + kWaves - 1) / kWaves;
+    const int64_t wgs = nx * H * num_seqs, slots = 2 * (int64_t)device_cus();
+    int64_t split = 1;
+    if (wgs > 0 && 2 * wgs <= slots) split = std::min<int64_t>(slots / wgs, prefill_tiles(max_seq_len) / kSplitTiles);
+    return {nx, std::max<int64_t>(1, split)};
+}
+static int64_t partial_bytes(const PrefillShape &p, int64_t num_seqs, int H) {
+    return p.split > 1 ? p.nx * p.split * H * num_seqs * kWaves * (int64_t)kPartFloats * 4 : 0;
+}
 
 }  // namespace rq
 
@@ -449,6 +569,14 @@ using namespace rq;
 extern "C" int64_t rq_int8_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads, int64_t max_seq_len) {
     if (num_seqs <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 0;
     return num_seqs * num_kv_heads * prefill_tiles(max_seq_len) * kImBytes;
+}
+
+extern "C" int64_t rq_prefill_split_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                                    int64_t max_q_len, int64_t max_seq_len) {
+    const int64_t images = rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len);
+    if (images == 0 || max_q_len <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0) return images;
+    return images + partial_bytes(prefill_shape(num_seqs, num_q_heads / num_kv_heads, num_kv_heads, max_q_len, max_seq_len),
+                                  num_seqs, num_kv_heads);
 }
 
 namespace {
@@ -519,6 +647,12 @@ int prefill_call(bool fused, int causal, const void *q, int32_t dtype, int64_t t
     a.causal = causal != 0;
     a.max_tiles = prefill_tiles(max_seq_len);
     a.ws = static_cast<uint8_t *>(workspace);
+    // key chunks when the workspace also holds their partials (after the tile images)
+    PrefillShape shape = prefill_shape(num_seqs, a.G, a.H, max_q_len, max_seq_len);
+    if (workspace_bytes < need + partial_bytes(shape, num_seqs, a.H)) shape.split = 1;
+    a.nx = (int)shape.nx;
+    a.split = (int)shape.split;
+    a.part = reinterpret_cast<float *>(a.ws + need);
     a.out = out;
     a.o_st = out_stride_tok;
     a.o_sh = out_stride_head;
@@ -528,8 +662,8 @@ int prefill_call(bool fused, int causal, const void *q, int32_t dtype, int64_t t
     else launch_pack<RQ_DTYPE_F16>(a, num_seqs, st);
     int rc = check_launch("prefill_pack_kernel");
     if (rc) return rc;
-    if (bf) launch_attn<RQ_DTYPE_BF16>(a, num_seqs, max_q_len, st);
-    else launch_attn<RQ_DTYPE_F16>(a, num_seqs, max_q_len, st);
+    if (bf) launch_attn<RQ_DTYPE_BF16>(a, num_seqs, st);
+    else launch_attn<RQ_DTYPE_F16>(a, num_seqs, st);
     return check_launch("prefill_attn_kernel");
 }
 

@@ -400,12 +400,17 @@ def fused_paged_rq_decode_launcher(q: torch.Tensor, kv_cache: torch.Tensor, bloc
     return launch
 
 
-def _prefill_workspace(dev, workspace, need: int, short_need: int) -> torch.Tensor:
+# At least the partials of any prefill call's key chunks (rq_prefill_split_workspace_bytes less its images).
+PREFILL_SPLIT_BYTES = 36 << 20
+
+
+def _prefill_workspace(dev, workspace, need: int, want: int) -> torch.Tensor:
     """Scratch of a prefill call: the caller's buffer if it holds the tile images (need), else the shared
-    one, large enough for the short-query kernels too when the call can take them."""
+    one, large enough (want) also for the short-query kernels or the partials of key chunks, whichever
+    the call can take."""
     if workspace is not None and workspace.numel() >= need:
         return workspace
-    return shared_workspace(dev, "prefill", max(need, short_need))
+    return shared_workspace(dev, "prefill", max(need, want))
 
 
 # ---------------------------------------------------------------------------
@@ -502,7 +507,8 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
     need = L.rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
     sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc)
-    ws = _prefill_workspace(dev, workspace, need, sneed)
+    want = sneed or L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
+    ws = _prefill_workspace(dev, workspace, need, want)
     short = sneed and ws.numel() >= sneed
     fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_int8_prefill, "rq_int8_prefill")
     rc = fn(
@@ -616,7 +622,8 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
     need = L.rq_paged_prefill_workspace_bytes(sl.numel(), num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
     sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc)
-    ws = _prefill_workspace(dev, workspace, need, sneed)
+    want = sneed or L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
+    ws = _prefill_workspace(dev, workspace, need, want)
     short = sneed and ws.numel() >= sneed
     fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_paged_prefill, "rq_paged_prefill")
     rc = fn(

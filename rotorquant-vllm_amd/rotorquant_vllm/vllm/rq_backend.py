@@ -117,6 +117,7 @@ _paged_attention_fn = None
 _paged_prefill_fn = None
 _unfused_decode_fn = None
 _shared_workspace = None
+PREFILL_SPLIT_BYTES = 0
 try:
     from rotorquant_vllm import _lib as _rq_lib
     from rotorquant_vllm.kernels import compress_store as _compress_store_fn
@@ -128,6 +129,7 @@ try:
     from rotorquant_vllm.kernels import fused_paged_rq_decode as _unfused_decode_fn
     from rotorquant_vllm.kernels import paged_decompress as _paged_decompress_fn
     from rotorquant_vllm.kernels import shared_workspace as _shared_workspace
+    from rotorquant_vllm.kernels import PREFILL_SPLIT_BYTES
 
     _rq_lib.load()
     _fused_paged_kernel_available = True
@@ -588,7 +590,7 @@ class RQAttentionImpl(_ImplBase):
         """Device tensors every launch reads (codebooks, R and its R^T splits), and the
         shared workspaces sized for the largest call this configuration allows
         (max_num_seqs sequences of max_model_len for decode, one max_model_len
-        sequence of tile images for prefill).  This runs at the first forward --
+        sequence of tile images and the partials of a prefill call's key chunks).  This runs at the first forward --
         vLLM's profiling run -- so later calls find their scratch allocated; the
         workspaces are shared by all layers of the process on this device and are
         never freed (rotorquant_vllm.kernels.shared_workspace)."""
@@ -608,7 +610,8 @@ class RQAttentionImpl(_ImplBase):
                 _shared_workspace(dev, "decode", lib.rq_fused_decode_workspace_bytes(
                     self._max_num_seqs, self.num_heads, self.head_size, cap))
             if self._fused_prefill_available or self._unfused_kernel_ok(compute_dtype, self.num_heads):
-                _shared_workspace(dev, "prefill", lib.rq_int8_prefill_workspace_bytes(1, self.num_kv_heads, cap))
+                _shared_workspace(dev, "prefill", lib.rq_int8_prefill_workspace_bytes(1, self.num_kv_heads, cap)
+                                  + PREFILL_SPLIT_BYTES)
         self._cg_buffers_ready = True
 
     def _layout_kw(self) -> dict:
@@ -660,6 +663,8 @@ class RQAttentionImpl(_ImplBase):
         [(b_start, b_end, max_seq_len, max_q_len)]."""
         lib = _rq_lib.load()
         budget = _shared_workspace(device, "prefill", 0).numel()
+        if budget > PREFILL_SPLIT_BYTES:  # room for the partials of a group's key chunks beside its images
+            budget -= PREFILL_SPLIT_BYTES
         cap = max_blocks * BS
         groups, start, mx, mq = [], b0, 0, 0
         for b in range(b0, len(lens)):

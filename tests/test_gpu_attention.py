@@ -192,6 +192,31 @@ def test_attention_short_queries_more_than_keys():
         assert excess <= 0 and cs >= 0.999, (err, excess, cs)
 
 
+@pytest.mark.parametrize("H,HQ,mode,dtype,causal", [(1, 4, "iso", torch.bfloat16, True), (2, 14, "planar", torch.float16, True),
+                                                    (1, 1, "iso", torch.bfloat16, False), (4, 32, "iso", torch.bfloat16, True)])
+def test_prefill_key_chunks(H, HQ, mode, dtype, causal):
+    """Few query blocks behind long prefixes: several workgroups per query block, each with a run of its tiles, and a
+    merge of their partials.  Chunk counts that do not divide the tiles, blocks with fewer tiles than
+    chunks, a sequence that ends inside the first chunk, waves above the diagonal in the last one; the same call with
+    scratch for the tile images alone runs unsplit."""
+    from rotorquant_vllm import _lib, kernels as K
+    q_lens = [33, 20, 0, 97]
+    ctx = [33 + 5000, 20 + 200, 17, 97 + 1601]
+    case = attn_case(120 + HQ, q_lens, ctx, H, HQ, Params(mode, 3, 4), dtype=dtype)
+    lib = _lib.load()
+    cap = case["bt"].shape[1] * case["BS"]
+    images = lib.rq_paged_prefill_workspace_bytes(4, H, cap)
+    assert lib.rq_prefill_split_workspace_bytes(4, HQ, H, 97, cap) > images, "the shape is one that splits"
+    check(case, f"chunks-{HQ}", causal=causal, entry="paged_prefill")
+    p = case["p"]
+    one = K.paged_prefill(_dev(case["q"]), _dev(case["cache"]), _dev(case["bt"]), _dev(case["lens"]), _dev(case["cu"]), 97, _dev(p.kc),
+                          _dev(p.vc), _dev(p.R), H, 128, 16, causal=causal, workspace=torch.empty(images, dtype=torch.uint8, device="cuda"))
+    torch.cuda.synchronize()
+    dt = str(dtype).replace("torch.", "")
+    err, excess, cs = check_tolerance(one.float().cpu().numpy(), ref(case, causal), dt, rot_block=p.blk)
+    assert excess <= 0 and cs >= 0.999, (err, excess, cs)
+
+
 def test_attention_graph_replay():
     """The call captured in a HIP graph: each replay, after the eager work between
     replays (new q and context lengths written into the captured buffers), equals
