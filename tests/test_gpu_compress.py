@@ -228,3 +228,34 @@ def test_compress_store_heads_not_dividing_workgroup(H):
     O.compress_store(ref, slots.numpy(), kp, kn, vp, vn)
     got = cache.cpu().numpy()
     assert np.array_equal(got, ref), f"{int((got != ref).sum())} bytes differ"
+
+
+@pytest.mark.parametrize("B,MB,NB", [(1, 1, 1), (3, 5, 31), (2, 16, 32), (7, 9, 33), (8, 512, 5000), (9, 456, 5000),
+                                     (4, 100, 8192), (4, 100, 8193)])
+def test_paged_decompress_indices(B, MB, NB):
+    """Compact ids, count and remapped table of small batches (one workgroup: up to 4096 table entries and 8192
+    blocks) and of the next larger ones (one kernel per step), against numpy: shared blocks, entries
+    out of range, lengths of zero, in mid-block and past the table."""
+    from rotorquant_vllm import kernels as K
+    H, D, BS = 1, 16, 4
+    rng = np.random.RandomState(B * 1000 + MB)
+    bt = rng.randint(-1, NB + 1, (B, MB)).astype(np.int32)  # -1 and NB: out of range
+    bt[:, 0] = NB - 1                                       # shared
+    lens = rng.randint(0, MB * BS + 1, B).astype(np.int32)
+    lens[0] = MB * BS + 7
+    if B > 1:
+        lens[1] = 0
+    cache = torch.zeros(NB, BS, 32, dtype=torch.uint8, device="cuda")
+    cb = torch.linspace(-1, 1, 8, device="cuda")
+    nb = np.minimum((lens + BS - 1) // BS, MB)
+    used = np.arange(MB)[None, :] < nb[:, None]
+    inside = (bt >= 0) & (bt < NB)
+    order = np.unique(bt[used & inside])
+    ids = np.zeros(NB, np.int32)
+    ids[order] = np.arange(len(order))
+    want = np.where(inside & np.isin(bt, order), ids[np.clip(bt, 0, NB - 1)], 0)
+    out = torch.empty(max(len(order), 1), BS, H, D, dtype=torch.bfloat16, device="cuda")
+    _, _, remap, count = K.paged_decompress(cache, torch.from_numpy(bt).cuda(), torch.from_numpy(lens).cuda(), H, D, cb, cb,
+                                            torch.bfloat16, out_k=out, out_v=torch.empty_like(out))
+    torch.cuda.synchronize()
+    assert int(count) == len(order) and np.array_equal(remap.cpu().numpy(), want)
