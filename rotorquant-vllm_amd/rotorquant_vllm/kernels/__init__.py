@@ -423,7 +423,7 @@ def _prefill_workspace(dev, workspace, need: int, want: int) -> torch.Tensor:
 _SHORT_WORKSPACE_LIMIT = 256 << 20
 
 
-def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc) -> int:
+def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc, out) -> int:
     """Workspace of rq_short_attention for this call, or 0 when the call does not take it.
 
     It is the faster one wherever it takes the call (at most four groups of 16 (token, query head)
@@ -434,6 +434,9 @@ def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_le
     if kc.numel() not in (8, 16) or vc.numel() not in (8, 16) or kc.data_ptr() % 16 or vc.data_ptr() % 16:
         return 0
     if kv_cache.data_ptr() % 16 or kv_cache.stride(0) % 16 or kv_cache.stride(1) % 16:
+        return 0
+    # output rows of other alignments: what the other kernels take or refuse
+    if out.data_ptr() % 8 or out.stride(0) % 4 or out.stride(1) % 4:
         return 0
     need = L.rq_short_attention_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
     return need if need <= _SHORT_WORKSPACE_LIMIT else 0
@@ -506,7 +509,7 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
     L = _lib.load()
     need = L.rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc)
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc, out)
     want = sneed or L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
     ws = _prefill_workspace(dev, workspace, need, want)
     short = sneed and ws.numel() >= sneed
@@ -569,7 +572,7 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale),
             out.data_ptr(), out.stride(0), out.stride(1))
     max_seq_len = bt.shape[1] * block_size
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc)
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc, out)
     if sneed:
         # scratch of this call alone, from the stream's allocator: the call stays usable on several
         # streams at once, as the workspace-free kernel is
@@ -621,7 +624,7 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
     L = _lib.load()
     need = L.rq_paged_prefill_workspace_bytes(sl.numel(), num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc)
+    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out)
     want = sneed or L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
     ws = _prefill_workspace(dev, workspace, need, want)
     short = sneed and ws.numel() >= sneed

@@ -154,3 +154,16 @@ def test_rotation_block_cache_is_per_tensor_object():
     b = s.view(128, 128)
     assert b.data_ptr() == a.data_ptr() and b._version == a._version
     assert K.rotation_block(b) == 4
+
+
+@pytest.mark.parametrize("offset,stride,taken", [(0, 128, True), (4, 128, True), (1, 128, False), (2, 128, False),
+                                                 (0, 130, False), (0, 132, True)])
+def test_short_queries_keep_the_other_kernels_output_alignment(offset, stride, taken):
+    """Output rows that are not 8-byte aligned (offset and stride in 2-byte elements) stay with the
+    kernels that took or refused them before."""
+    from rotorquant_vllm import kernels as K
+
+    out = torch.zeros(4 + 3 * 8 * stride, dtype=torch.float16).as_strided((3, 8, 128), (8 * stride, stride, 1), offset)
+    cache = torch.zeros(4, 16, 512, dtype=torch.uint8)
+    c = torch.zeros(8)
+    assert (K._short_attention_bytes(_lib.load(), 8, 2, 1, 3, 64, cache, c, c, out) > 0) == taken
