@@ -1,4 +1,4 @@
-"""GPU parity: int8-MFMA causal prefill vs the float64 oracle.
+"""GPU parity: causal prefill vs the float64 oracle.
 
 Tolerance as for decode (rq_testlib.check_tolerance): cos >= 0.999 and
 |got - ref| <= max(2e-2, ulp(x_d) + 2 ulp(rotation-block max)); unit-scale
