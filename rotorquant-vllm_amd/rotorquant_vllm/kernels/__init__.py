@@ -421,12 +421,17 @@ def _prefill_workspace(dev, workspace, need: int, want: int) -> torch.Tensor:
 # partials take 0.5 KB per (token, head) column and workgroup, the descriptors 8.5
 # bytes per key of the block table's capacity and column group).
 _SHORT_WORKSPACE_LIMIT = 256 << 20
+# Block-table capacity up to which paged_attention keeps its one launch (up to four tiles of 64 keys a
+# workgroup) instead of the three of the short-query kernels.  32 / 8 heads, up to 8 tokens each, three
+# launches against one: 4 sequences of up to 64 keys 19.8 / 10.3 us, 128 20.0 / 13.1, 256 20.6 / 19.9;
+# 64 sequences 39.4 / 11.5, 42.8 / 16.6, 48.8 / 26.4 (their descriptors and partials grow with the batch).
+_ONE_LAUNCH_KEYS = 256
 
 
 def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc, out) -> int:
     """Workspace of rq_short_attention for this call, or 0 when the call does not take it.
 
-    It is the faster one wherever it takes the call (at most four groups of 16 (token, query head)
+    It is the faster one for contexts of more than a few tiles (at most four groups of 16 (token, query head)
     columns per kv head): 32 sequences of 600-8000 keys, 32 / 8 heads, up to 8 tokens each,
     437 us in rq_paged_attention, 87 us here."""
     if not 1 <= max_q_len <= 16 or num_kv_heads > 64 or max_seq_len < 1 or kv_cache.shape[0] < 1:
@@ -572,7 +577,9 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale),
             out.data_ptr(), out.stride(0), out.stride(1))
     max_seq_len = bt.shape[1] * block_size
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc, out)
+    sneed = 0
+    if max_seq_len > _ONE_LAUNCH_KEYS:
+        sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc, out)
     if sneed:
         # scratch of this call alone, from the stream's allocator: the call stays usable on several
         # streams at once, as the workspace-free kernel is
