@@ -1194,7 +1194,9 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
             o1 += f * x.y;
         }
     }
-    const float inv = nch > 0 && lsum > 0.f ? 1.f / lsum : 0.f;  // no key seen -> zeros (reference: acc 0, l 1)
+    // No key seen -> zeros (reference: acc 0, l 1).  With SHORT a token may see none of its entry's keys; a decode
+    // sees every key, so a sum of 0 means that all its scores overflowed to -inf, which has no softmax: 0 / 0 = NaN.
+    const float inv = nch > 0 && (!SHORT || lsum > 0.f) ? 1.f / lsum : 0.f;
     orot[2 * lane] = Elem<DT>::to_f32(Elem<DT>::from_f32(o0 * inv));
     orot[2 * lane + 1] = Elem<DT>::to_f32(Elem<DT>::from_f32(o1 * inv));
     __builtin_amdgcn_wave_barrier();

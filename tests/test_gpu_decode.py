@@ -187,6 +187,30 @@ def test_decode_closed_forms():
         assert excess <= 0 and cs >= 0.9999
 
 
+@pytest.mark.parametrize("L", [1, 333, 20000])
+def test_decode_scores_that_all_overflow_are_nan(L):
+    """Every score of a sequence below fp32's range (-inf): softmax has no value, and the output is NaN, not
+    the zeros of an empty context.  One key, one tile per workgroup, and ranges by weight; the other sequence of the
+    batch keeps its values."""
+    p = Params("iso", 3, 3)
+    H = HQ = 2
+    k_norm = 64 * H  # byte offset of the K norms in a slot
+    case = decode_case(46, 2, H, HQ, [L, 40], p=p)
+    cache, blocks = case["cache"], case["bt"][0][:-(-L // 16)]
+    alone = dict(case, bt=case["bt"][1:], lens=case["lens"][1:], q=case["q"][1:])
+    want = ref_decode(alone)
+    cache[blocks, :, :k_norm] = cache[blocks[0], 0, :k_norm]  # one K vector for all keys of the sequence
+    cache[blocks, :, k_norm:k_norm + 4 * H] = np.frombuffer(np.full(H, 1e38, np.float32).tobytes(), np.uint8)
+    idx = cache[blocks[0], 0, :k_norm].reshape(H, 64)
+    sign = np.sign(p.kc.numpy()[np.stack([idx >> 4, idx & 15], -1).reshape(H, 128)])
+    # q_rot = q R^T has the opposite sign of K in every dim: each product is -inf or far below 0
+    case["q"][0] = (torch.from_numpy(-1e4 * sign).float() @ p.R).to(case["q"].dtype)
+    got = run_decode(case)
+    assert np.isnan(got[0]).all()
+    _, excess, cs = check_tolerance(got[1:], want, "bfloat16", rot_block=p.blk)
+    assert excess <= 0 and cs >= MIN_COS
+
+
 def test_decode_deterministic_and_batch_consistent():
     """The same batch decoded twice gives identical bits.  A sequence decoded alone
     and inside a batch of long sequences agrees within the parity tolerance (work
