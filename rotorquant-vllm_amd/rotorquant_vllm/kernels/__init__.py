@@ -404,13 +404,20 @@ def fused_paged_rq_decode_launcher(q: torch.Tensor, kv_cache: torch.Tensor, bloc
 PREFILL_SPLIT_BYTES = 36 << 20
 
 
-def _prefill_workspace(dev, workspace, need: int, want: int) -> torch.Tensor:
-    """Scratch of a prefill call: the caller's buffer if it holds the tile images (need), else the shared
-    one, large enough (want) also for the short-query kernels or the partials of key chunks, whichever
-    the call can take."""
+def _prefill_workspace(dev, workspace, need: int, split: int, short: int) -> tuple[torch.Tensor, bool]:
+    """(scratch, whether the short-query kernels run on it) of a prefill call.
+
+    need, split: bytes of the tile images, and of these and the partials of key chunks; short: bytes of the
+    short-query kernels, 0 when the call does not take them.  The caller's buffer if it holds the tile
+    images; else for short queries the shared buffer as far as it goes and otherwise scratch of this call from the
+    stream's allocator (the shared buffer never shrinks: a server's batches of drafts, each a little larger
+    than the last, would leave the sum of their sizes behind); else the shared buffer."""
     if workspace is not None and workspace.numel() >= need:
-        return workspace
-    return shared_workspace(dev, "prefill", max(need, want))
+        return workspace, 0 < short <= workspace.numel()
+    if short:
+        shared = shared_workspace(dev, "prefill", 0)
+        return (shared if shared.numel() >= short else torch.empty(short, dtype=torch.uint8, device=dev)), True
+    return shared_workspace(dev, "prefill", max(need, split)), False
 
 
 # ---------------------------------------------------------------------------
@@ -515,9 +522,8 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
     need = L.rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
     sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc, out)
-    want = sneed or L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
-    ws = _prefill_workspace(dev, workspace, need, want)
-    short = sneed and ws.numel() >= sneed
+    split = L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
+    ws, short = _prefill_workspace(dev, workspace, need, split, sneed)
     fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_int8_prefill, "rq_int8_prefill")
     rc = fn(
         q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
@@ -632,9 +638,8 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
     need = L.rq_paged_prefill_workspace_bytes(sl.numel(), num_kv_heads, max_seq_len)
     short_len = min(max_seq_len, bt.shape[1] * block_size)
     sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out)
-    want = sneed or L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
-    ws = _prefill_workspace(dev, workspace, need, want)
-    short = sneed and ws.numel() >= sneed
+    split = L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
+    ws, short = _prefill_workspace(dev, workspace, need, split, sneed)
     fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_paged_prefill, "rq_paged_prefill")
     rc = fn(
         q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),

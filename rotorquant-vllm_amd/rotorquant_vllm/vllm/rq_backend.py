@@ -591,9 +591,10 @@ class RQAttentionImpl(_ImplBase):
         shared workspaces sized for the largest call this configuration allows
         (max_num_seqs sequences of max_model_len for decode, one max_model_len
         sequence of tile images and the partials of a prefill call's key chunks).  This runs at the first forward --
-        vLLM's profiling run -- so later calls find their scratch allocated; the
+        vLLM's profiling run -- so later decodes and prefills find their scratch allocated; the
         workspaces are shared by all layers of the process on this device and are
-        never freed (rotorquant_vllm.kernels.shared_workspace)."""
+        never freed (rotorquant_vllm.kernels.shared_workspace).  Batches of drafts (2 to 16 tokens per sequence)
+        may need more: up to 256 MB, allocated for the call."""
         dev = kv_cache.device
         self._dev_kc = self._k_quantizer.centroids.to(dev, torch.float32).contiguous()
         self._dev_vc = self._v_quantizer.centroids.to(dev, torch.float32).contiguous()
