@@ -1032,7 +1032,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
     #pragma unroll
         for (int i = 0; i < 8; ++i) {
             p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc, -m_run));
-            l_run += p[i];
+            if constexpr (!SHORT) l_run += p[i];
         }
 
         // ---- O^T += V^T P^T ---------------------------------------------------
@@ -1040,6 +1040,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(decode_wave
         // (p, 0) in columns < 8 and (0, p) in columns >= 8, or (WIDE) both.
         const uint32_t x01 = pack2<RQ_DTYPE_F16>(p[0], p[1]), x23 = pack2<RQ_DTYPE_F16>(p[2], p[3]);
         const uint32_t x45 = pack2<RQ_DTYPE_F16>(p[4], p[5]), x67 = pack2<RQ_DTYPE_F16>(p[6], p[7]);
+        // Short queries divide by the sum of the rounded weights of the numerator, as rq_paged_attention does: the
+        // roundings then cancel where the keys' V agree (v_dot2_f32_f16: exact products, fp32 sums).
+        if constexpr (SHORT) {
+            typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+            const f16x2 one = {(_Float16)1.f, (_Float16)1.f};
+    #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t x = i == 0 ? x01 : i == 1 ? x23 : i == 2 ? x45 : x67;
+                l_run = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, x), one, l_run, false);
+            }
+        }
         if constexpr (!WIDE) {
             const bool hi_col = (lane_now() & 8) != 0;
             const uint32_t se = hi_col ? 0x01000c0cu : 0x0c0c0100u;  // element 0 -> (x, 0) or (0, x)
