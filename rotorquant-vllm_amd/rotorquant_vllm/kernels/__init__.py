@@ -16,10 +16,13 @@ the C ABI (include/rq_abi.h).  Differences, all deliberate:
 * paged_attention has no op-level counterpart: it is the backend's non-fused
   path (paged decompress + flash_attn_varlen_func + the two rotations,
   rq_backend.py:937-1036) as one launch; paged_prefill is the same arithmetic
-  in two launches (each 64-key tile decoded once), for long queries.
+  with each 64-key tile decoded once, for long queries (two launches, or three
+  where few query blocks are spread over the GPU by key chunks).  Calls of at most 16
+  tokens per sequence run on the decode kernels (three launches) where that is faster.
 """
 from __future__ import annotations
 
+import functools
 import math
 import weakref
 
@@ -426,21 +429,58 @@ def _prefill_workspace(dev, workspace, need: int, split: int, short: int) -> tup
 
 # Workspace above which a call keeps the kernels that need none or less of it (the
 # partials take 0.5 KB per (token, head) column and workgroup, the descriptors 8.5
-# bytes per key of the block table's capacity and column group).
+# bytes per key of the bound on the lengths and column group).
 _SHORT_WORKSPACE_LIMIT = 256 << 20
-# Block-table capacity up to which paged_attention keeps its one launch (up to four tiles of 64 keys a
-# workgroup) instead of the three of the short-query kernels.  32 / 8 heads, up to 8 tokens each, three
-# launches against one: 4 sequences of up to 64 keys 19.8 / 10.3 us, 128 20.0 / 13.1, 256 20.6 / 19.9;
-# 64 sequences 39.4 / 11.5, 42.8 / 16.6, 48.8 / 26.4 (their descriptors and partials grow with the batch).
-_ONE_LAUNCH_KEYS = 256
+
+# Which kernels take a call of at most 16 tokens per sequence: the ones with the least estimated GPU time (us), as
+# functions of the heads, the number of sequences and the bound on their lengths.  Fitted to captured calls on MI355X, iso 3-bit:
+# 4 / 16 / 64 / 128 sequences, 2 to 16 tokens, 64 to 1024 keys, 8 x 4, 1 x 4, 4 x 7, 8 x 1 and 2 x 8 (kv heads x
+# query heads of each).  32 / 8 heads, 8 tokens:
+#   sequences x keys       one launch   short   prefill kernels (us)
+#   4 x 64 / 256 / 1024    9 / 19 / 59   18 / 20 / 31   13 / 18 / 33
+#   64 x 64 / 256 / 1024   12 / 26 / 76   45 / 55 / 77   20 / 39 / 122
+#   128 x 64 / 256 / 1024   25 / 49 / 148   69 / 81 / 129   34 / 70 / 277
+
+
+def _one_launch_us(H, G, num_seqs, max_q_len, keys) -> float:
+    """rq_paged_attention: a workgroup per sequence, kv head and part of a group above 8 heads goes through the 64-key tiles
+    one after the other, about 400 workgroups side by side."""
+    parts = 1 if G <= 8 else next(p for p in range(2, G + 1) if G % p == 0 and G // p <= 8)
+    return (6 + 3.4 * -(-keys // 64)) * max(1.0, num_seqs * H * parts / 400) * (1.1 if G >= 7 else 1.0)
+
+
+def _short_us(H, G, num_seqs, max_q_len, keys) -> float:
+    """rq_short_attention: three launches; the columns to merge, the partials of up to a workgroup each, the tiles of 32 keys."""
+    tokens = min(16 // G, max_q_len)
+    entries = num_seqs * -(-max_q_len // tokens)
+    columns, tiles = H * G * tokens, entries * -(-keys // 32)
+    return 15.6 + 1e-3 * (1.09 * entries * columns + 0.25 * min(tiles, 512 + entries) * columns + 0.87 * tiles * H)
+
+
+def _prefill_us(H, G, num_seqs, max_q_len, keys) -> float:
+    """rq_paged_prefill / rq_int8_prefill: every tile unpacked to memory, then a workgroup per four (query block, head)
+    units, or with few of them one per chunk of the tiles."""
+    workgroups, tiles = -(-G // 4) * H * num_seqs, -(-keys // 64)
+    split = max(1, min(512 // workgroups, tiles // 8)) if 2 * workgroups <= 512 else 1
+    chain = max(4, -(-tiles // split)) + 2 if split > 1 else tiles
+    return 12.9 + 1.15 * chain * max(1.0, workgroups / 512) + 0.011 * H * num_seqs * tiles + max(0, H * num_seqs * tiles - 4096) * 2e-3
+
+
+@functools.lru_cache(maxsize=4096)  # (by sizes alone; a few microseconds on the launch path)
+def _faster_kernels(H, G, num_seqs, max_q_len, keys, prefill_kernels) -> str:
+    """ "short" (rq_short_attention), "one" (rq_paged_attention) or "" (the caller's own: the prefill kernels with
+    prefill_kernels, else rq_paged_attention)."""
+    shape = (H, G, num_seqs, max_q_len, keys)
+    # (10 % for its scratch, and against estimates that are off)
+    one, short = _one_launch_us(*shape), 1.1 * _short_us(*shape)
+    if prefill_kernels and _prefill_us(*shape) < min(one, short):
+        return ""
+    return "short" if short < one else "one" if prefill_kernels else ""
 
 
 def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc, out) -> int:
-    """Workspace of rq_short_attention for this call, or 0 when the call does not take it.
-
-    It is the faster one for contexts of more than a few tiles (at most four groups of 16 (token, query head)
-    columns per kv head): 32 sequences of 600-8000 keys, 32 / 8 heads, up to 8 tokens each,
-    437 us in rq_paged_attention, 87 us here."""
+    """Workspace of rq_short_attention for this call, or 0 when the call does not take it (at most 16 tokens in at most four
+    groups of 16 (token, query head) columns per kv head)."""
     if not 1 <= max_q_len <= 16 or num_kv_heads > 64 or max_seq_len < 1 or kv_cache.shape[0] < 1:
         return 0
     if kc.numel() not in (8, 16) or vc.numel() not in (8, 16) or kc.data_ptr() % 16 or vc.data_ptr() % 16:
@@ -452,6 +492,18 @@ def _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_le
         return 0
     need = L.rq_short_attention_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
     return need if need <= _SHORT_WORKSPACE_LIMIT else 0
+
+
+def _short_route(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc, out, prefill_kernels) -> tuple[str, int]:
+    """(_faster_kernels of a call, workspace of rq_short_attention); the caller's own for calls that one does not take."""
+    G = H_Q // num_kv_heads
+    if not 1 <= max_q_len <= 16 or num_seqs < 1 or not 1 <= G <= 16:
+        return "", 0
+    kernels = _faster_kernels(num_kv_heads, G, num_seqs, max_q_len, max_seq_len, prefill_kernels)
+    if not kernels:
+        return "", 0
+    need = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, max_seq_len, kv_cache, kc, vc, out)
+    return (kernels, need) if need else ("", 0)
 
 
 # ---------------------------------------------------------------------------
@@ -520,19 +572,26 @@ def fused_paged_rq_int8_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_t
         max_seq_len = bt.shape[1] * block_size
     L = _lib.load()
     need = L.rq_int8_prefill_workspace_bytes(num_seqs, num_kv_heads, max_seq_len)
+    sl = seq_lens.contiguous()
+    queries = (q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(), num_seqs, max_q_len)
+    cache = (kv_cache.data_ptr(), kv_cache.shape[0], block_size, kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim,
+             _layout(dense3), bt.data_ptr(), bt.shape[1], bt.stride(0), sl.data_ptr())
+    tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale), out.data_ptr(), out.stride(0),
+            out.stride(1))
     short_len = min(max_seq_len, bt.shape[1] * block_size)
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc, out)
-    split = L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
+    route, sneed = _short_route(L, H_Q, num_kv_heads, num_seqs, max_q_len, short_len, kv_cache, kc, vc, out, True)
+    if route == "one":
+        rc = L.rq_paged_attention(*queries, 1, *cache, *tail, _lib.stream_ptr(dev))
+        _lib.check(rc, "rq_paged_attention")
+        return out
+    split = 0 if sneed else L.rq_prefill_split_workspace_bytes(num_seqs, H_Q, num_kv_heads, max_q_len, max_seq_len)
     ws, short = _prefill_workspace(dev, workspace, need, split, sneed)
-    fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_int8_prefill, "rq_int8_prefill")
-    rc = fn(
-        q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
-        num_seqs, max_q_len, *((1,) if short else ()), kv_cache.data_ptr(), kv_cache.shape[0], block_size, kv_cache.stride(0),
-        kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1], bt.stride(0),
-        seq_lens.contiguous().data_ptr(), short_len if short else max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(),
-        R.data_ptr(), blk, float(sm_scale), out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws.numel(),
-        _lib.stream_ptr(dev))
-    _lib.check(rc, name)
+    if short:
+        rc = L.rq_short_attention(*queries, 1, *cache, short_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+        _lib.check(rc, "rq_short_attention")
+        return out
+    rc = L.rq_int8_prefill(*queries, *cache, max_seq_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+    _lib.check(rc, "rq_int8_prefill")
     return out
 
 
@@ -544,7 +603,8 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
                     cu_seqlens_q: torch.Tensor, max_q_len: int, k_centroids: torch.Tensor,
                     v_centroids: torch.Tensor, rotation: torch.Tensor, num_kv_heads: int, head_dim: int,
                     block_size: int, sm_scale: float | None = None, causal: bool = True,
-                    out: torch.Tensor | None = None, dense3: bool = False) -> torch.Tensor:
+                    out: torch.Tensor | None = None, dense3: bool = False,
+                    max_seq_len: int | None = None) -> torch.Tensor:
     """Attention of the new query tokens over the packed cache, q and output in original space.
 
     The reference's non-fused path (rq_backend.py:937-1036: q_rot = q R^T cast to
@@ -555,7 +615,10 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     (num_seqs,) int32 context lengths including the new tokens; max_q_len: a host
     int bounding every q_len (it sizes the grid).  Query i of sequence b sits at
     position seq_lens[b] - q_len_b + i.  dense3: the cache holds the dense 3-bit
-    index layout.
+    index layout.  max_seq_len: a host int bounding every seq_lens entry (default: the
+    block table's capacity), by which calls of at most 16 tokens per sequence
+    choose between the two; a table much wider than the contexts is taken at its width
+    without it.
     """
     num_tokens, H_Q, D = q.shape
     assert D == head_dim
@@ -582,15 +645,14 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
             bt.stride(0), sl.data_ptr())
     tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale),
             out.data_ptr(), out.stride(0), out.stride(1))
-    max_seq_len = bt.shape[1] * block_size
-    sneed = 0
-    if max_seq_len > _ONE_LAUNCH_KEYS:
-        sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), max_seq_len, kv_cache, kc, vc, out)
-    if sneed:
+    capacity = bt.shape[1] * block_size
+    short_len = capacity if max_seq_len is None else min(max_seq_len, capacity)
+    route, sneed = _short_route(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out, False)
+    if route == "short":
         # scratch of this call alone, from the stream's allocator: the call stays usable on several
         # streams at once, as the workspace-free kernel is
         ws = torch.empty(sneed, dtype=torch.uint8, device=dev)
-        rc = L.rq_short_attention(*head, max_seq_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
+        rc = L.rq_short_attention(*head, short_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
         _lib.check(rc, "rq_short_attention")
         return out
     rc = L.rq_paged_attention(*head, *tail, _lib.stream_ptr(dev))
@@ -636,18 +698,21 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
         max_seq_len = bt.shape[1] * block_size
     L = _lib.load()
     need = L.rq_paged_prefill_workspace_bytes(sl.numel(), num_kv_heads, max_seq_len)
+    queries = (q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
+               sl.numel(), int(max_q_len), 1 if causal else 0)
+    cache = (kv_cache.data_ptr(), kv_cache.shape[0], block_size, kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim,
+             _layout(dense3), bt.data_ptr(), bt.shape[1], bt.stride(0), sl.data_ptr())
+    tail = (kc.data_ptr(), kc.numel(), vc.data_ptr(), vc.numel(), R.data_ptr(), blk, float(sm_scale), out.data_ptr(), out.stride(0),
+            out.stride(1))
     short_len = min(max_seq_len, bt.shape[1] * block_size)
-    sneed = _short_attention_bytes(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out)
-    split = L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
+    route, sneed = _short_route(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out, True)
+    if route == "one":
+        rc = L.rq_paged_attention(*queries, *cache, *tail, _lib.stream_ptr(dev))
+        _lib.check(rc, "rq_paged_attention")
+        return out
+    split = 0 if sneed else L.rq_prefill_split_workspace_bytes(sl.numel(), H_Q, num_kv_heads, int(max_q_len), max_seq_len)
     ws, short = _prefill_workspace(dev, workspace, need, split, sneed)
     fn, name = (L.rq_short_attention, "rq_short_attention") if short else (L.rq_paged_prefill, "rq_paged_prefill")
-    rc = fn(
-        q.data_ptr(), _lib.dtype_code(q.dtype), num_tokens, H_Q, q.stride(0), q.stride(1), cu.data_ptr(),
-        sl.numel(), int(max_q_len), 1 if causal else 0, kv_cache.data_ptr(), kv_cache.shape[0], block_size,
-        kv_cache.stride(0), kv_cache.stride(1), num_kv_heads, head_dim, _layout(dense3), bt.data_ptr(), bt.shape[1],
-        bt.stride(0), sl.data_ptr(), short_len if short else max_seq_len, kc.data_ptr(), kc.numel(), vc.data_ptr(),
-        vc.numel(), R.data_ptr(),
-        blk, float(sm_scale), out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws.numel(),
-        _lib.stream_ptr(dev))
+    rc = fn(*queries, *cache, short_len if short else max_seq_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
     _lib.check(rc, name)
     return out

@@ -760,15 +760,20 @@ class RQAttentionImpl(_ImplBase):
         BS = kv_cache.shape[1]
         causal = bool(getattr(md, "causal", True))
         out = output[:num_actual_tokens]
+        sl_cpu = getattr(md, "rq_seq_lens_cpu", None)
         if int(max_q) <= RQ_UNFUSED_SHORT_Q or _paged_prefill_fn is None or _shared_workspace is None:
-            _paged_attention_fn(q, kv_cache, md.block_table, md.seq_lens, md.query_start_loc, int(max_q), kc, vc, R,
-                                self.num_kv_heads, self.head_size, BS, sm_scale=self.scale, causal=causal, out=out,
-                                **self._layout_kw())
+            # The host's longest context, where it is known, picks the kernels; a captured call is replayed over
+            # longer ones, so it goes by the block table's capacity.
+            longest = None
+            if sl_cpu is not None and sl_cpu.numel() and not (q.is_cuda and torch.cuda.is_current_stream_capturing()):
+                longest = int(sl_cpu.max())
+            _call_hook(_paged_attention_fn, q, kv_cache, md.block_table, md.seq_lens, md.query_start_loc, int(max_q), kc,
+                       vc, R, self.num_kv_heads, self.head_size, BS, sm_scale=self.scale, causal=causal, out=out,
+                       max_seq_len=longest, **self._layout_kw())
             return output
         if qsl_cpu is None:
             qsl_cpu = getattr(md, "rq_query_start_loc_cpu", None)
             qsl_cpu = qsl_cpu if qsl_cpu is not None else md.query_start_loc.cpu()
-        sl_cpu = getattr(md, "rq_seq_lens_cpu", None)
         qsl = qsl_cpu.tolist()
         lens = (sl_cpu if sl_cpu is not None else md.seq_lens.cpu()).tolist()
         B = len(lens)
@@ -784,9 +789,9 @@ class RQAttentionImpl(_ImplBase):
         while ns < B and q_lens[ns] <= RQ_UNFUSED_SHORT_Q:
             ns += 1
         if ns > nd:
-            _paged_attention_fn(q, kv_cache, bt[nd:ns], md.seq_lens[nd:ns], md.query_start_loc[nd:ns + 1],
-                                max(q_lens[nd:ns]), kc, vc, R, self.num_kv_heads, self.head_size, BS,
-                                sm_scale=self.scale, causal=causal, out=out, **self._layout_kw())
+            _call_hook(_paged_attention_fn, q, kv_cache, bt[nd:ns], md.seq_lens[nd:ns], md.query_start_loc[nd:ns + 1],
+                       max(q_lens[nd:ns]), kc, vc, R, self.num_kv_heads, self.head_size, BS, sm_scale=self.scale,
+                       causal=causal, out=out, max_seq_len=max(lens[nd:ns]), **self._layout_kw())
         for g0, g1, mx, mq in self._prefill_groups(lens, q_lens, ns, BS, bt.shape[1], query.device):
             _paged_prefill_fn(q, kv_cache, bt[g0:g1], md.seq_lens[g0:g1], md.query_start_loc[g0:g1 + 1], mq, kc, vc,
                               R, self.num_kv_heads, self.head_size, BS, sm_scale=self.scale, causal=causal, out=out,

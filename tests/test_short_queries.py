@@ -64,7 +64,77 @@ def test_drafts_do_not_grow_the_shared_prefill_buffer(launches, entry):
     L = _lib.load()
     buf = K.shared_workspace("cpu", "prefill", L.rq_int8_prefill_workspace_bytes(1, H, longest) + K.PREFILL_SPLIT_BYTES)
     for seqs in range(1, 129, 9):
-        call(entry, seqs, H, HQ, 8, 200, longest, max_seq_len=1200)
+        call(entry, seqs, H, HQ, 8, 200, longest, max_seq_len=3000)
     assert K.shared_workspace("cpu", "prefill", 0) is buf and not K._ws_retired
     assert {x.name for x in launches} == {"rq_short_attention"}
     assert max(x.scratch for x in launches) > buf.numel(), "some batch needs more than the buffer"
+
+
+# (sequences, kv heads, query heads, tokens, keys) -> kernels of paged_attention and of the prefill wrappers; both sides measured
+# (us, one launch / short / prefill kernels) at the points of the sweep that the estimates were fitted to.
+ROUTES = [
+    ((4, 8, 32, 8, 64), "rq_paged_attention", "rq_paged_attention"),      # 9 / 18 / 13
+    ((4, 8, 32, 8, 512), "rq_short_attention", "rq_short_attention"),     # 33 / 23 / 24
+    ((16, 8, 32, 8, 256), "rq_paged_attention", "rq_paged_attention"),    # 19 / 33 / 25
+    ((64, 8, 32, 8, 64), "rq_paged_attention", "rq_paged_attention"),     # 12 / 45 / 20
+    ((64, 8, 32, 8, 512), "rq_paged_attention", "rq_paged_attention"),    # 44 / 61 / 58
+    ((64, 8, 32, 2, 512), "rq_short_attention", "rq_short_attention"),    # 44 / 33 / 59
+    ((128, 8, 32, 8, 256), "rq_paged_attention", "rq_paged_attention"),   # 49 / 81 / 70
+    ((128, 8, 8, 4, 128), "rq_short_attention", "rq_short_attention"),    # 31 / 24 / 44
+    ((64, 4, 28, 4, 64), "rq_paged_attention", "rq_paged_attention"),     # 10 / 28 / 24
+    ((4, 8, 32, 16, 512), "rq_short_attention", "prefill"),               # 33 / 32 / 24
+    ((32, 8, 32, 8, 8000), "rq_short_attention", "rq_short_attention"),   # 431 / 83
+    ((1, 8, 32, 16, 100000), "rq_short_attention", "rq_short_attention"),
+    ((1, 1, 1, 1, 1), "rq_paged_attention", "rq_paged_attention"),
+]
+
+
+@pytest.mark.parametrize("shape,attention,prefill", ROUTES)
+def test_short_queries_take_the_faster_kernels(launches, shape, attention, prefill):
+    """By sequences, heads, tokens and the bound on the lengths: the block table's capacity, or max_seq_len where it is
+    given, whatever the table's width."""
+    keys = shape[-1]
+    own = {"fused_paged_rq_int8_prefill": "rq_int8_prefill", "paged_prefill": "rq_paged_prefill"}
+    call("paged_attention", *shape)
+    call("paged_attention", *shape, table_keys=131072, max_seq_len=keys)
+    assert [x.name for x in launches] == [attention] * 2
+    for entry in PREFILLS:
+        launches.clear()
+        call(entry, *shape)
+        call(entry, *shape, table_keys=131072, max_seq_len=keys)
+        assert [x.name for x in launches] == [own[entry] if prefill == "prefill" else prefill] * 2
+    for x in launches:
+        assert x.max_seq_len is None or keys <= x.max_seq_len < keys + 2 * BS
+
+
+@pytest.mark.parametrize("entry", ["paged_attention"] + PREFILLS)
+def test_calls_outside_the_short_kernels_keep_their_own(launches, entry):
+    """Longer queries, more groups of columns than the kernels take, scratch over the limit, no sequences."""
+    own = {"paged_attention": "rq_paged_attention", "fused_paged_rq_int8_prefill": "rq_int8_prefill", "paged_prefill": "rq_paged_prefill"}[entry]
+    for shape in ((4, 8, 32, 17, 4000), (4, 1, 9, 5, 4000), (4, 8, 64, 9, 4000), (128, 8, 32, 16, 1024), (0, 8, 32, 4, 4000)):
+        call(entry, *shape)
+    assert [x.name for x in launches] == [own] * 5
+
+
+@pytest.mark.parametrize("host_copies", [True, False])
+def test_backend_bounds_short_calls_by_the_host_lengths(monkeypatch, host_copies):
+    """The non-fused path gives paged_attention the longest context of its sequences where the metadata holds it on the
+    host: all sequences of a batch of short queries, or the short ones of a mixed batch."""
+    from rotorquant_vllm.vllm import rq_backend as B
+    from test_dispatch import _bare_impl, _mixed_metadata
+    seen = []
+
+    def attention(q, kv_cache, block_table, seq_lens, cu, max_q_len, *a, out=None, max_seq_len=None, **k):
+        seen.append((seq_lens.tolist(), max_seq_len))
+        return out
+
+    monkeypatch.setattr(B, "_paged_attention_fn", attention)
+    monkeypatch.setattr(B, "_paged_prefill_fn", lambda *a, out=None, **k: out)
+    monkeypatch.setattr(B, "_unfused_decode_fn", lambda *a, out=None, **k: out)
+    monkeypatch.setattr(K, "_ws_cache", {})
+    impl, cache = _bare_impl(False, False), torch.zeros(40, 16, 2048, dtype=torch.uint8)
+    for q_lens, lens in (([2, 1, 16], [500, 30, 900]), ([1, 3, 40], [500, 30, 300])):
+        md = _mixed_metadata(q_lens, lens, host_copies=host_copies)
+        query = torch.zeros(sum(q_lens), 32, 128, dtype=torch.bfloat16)
+        impl.forward(None, query, None, None, cache, md, output=torch.zeros_like(query))
+    assert seen == [([500, 30, 900], 900 if host_copies else None), ([30], 30)]
