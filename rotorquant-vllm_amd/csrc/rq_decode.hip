@@ -1342,14 +1342,15 @@ static void launch_decode_bits(DecodeArgs &a, size_t lds, int kb, int vb, bool d
 // Workspace layout (256-byte aligned regions).
 struct DecodeWorkspace {
     int64_t part_acc, part_ml, qops, descs, tile_prefix, n_tiles, total;
-    DecodeWorkspace(int64_t num_seqs, int64_t num_q_heads, int64_t max_seq_len) {
+    // qop_heads: kv heads that hold query operands (16 columns each), or a bound on them
+    DecodeWorkspace(int64_t num_seqs, int64_t num_q_heads, int64_t qop_heads, int64_t max_seq_len) {
         auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
         const int64_t slots = (int64_t)decode_slot_factor(num_q_heads) * device_cus() + num_seqs;
         const int64_t max_tiles = num_seqs * ((max_seq_len + kTile - 1) / kTile);
         part_acc = 0;
         part_ml = al(part_acc + slots * num_q_heads * kD * 4);
         qops = al(part_ml + slots * num_q_heads * 2 * 4);
-        descs = al(qops + num_seqs * num_q_heads * 64 * 16 * 4);  // kv heads <= query heads
+        descs = al(qops + num_seqs * qop_heads * 64 * 16 * 4);
         tile_prefix = al(descs + max_tiles * (int64_t)sizeof(TileDesc));
         n_tiles = al(tile_prefix + num_seqs * 8);  // NT (int) at +0, range-split multiplier (uint64) at +8
         total = al(n_tiles + 16);
@@ -1363,7 +1364,8 @@ using namespace rq;
 extern "C" int64_t rq_fused_decode_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t head_dim,
                                                    int64_t max_seq_len) {
     (void)head_dim;
-    return DecodeWorkspace(num_seqs, num_q_heads, std::max<int64_t>(max_seq_len, 1)).total;
+    // (the kv heads are not among the arguments: at most the query heads)
+    return DecodeWorkspace(num_seqs, num_q_heads, num_q_heads, std::max<int64_t>(max_seq_len, 1)).total;
 }
 
 // rq_short_attention's queries: cu_q per sequence, column groups of tpg tokens, vg per sequence.
@@ -1523,8 +1525,8 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     // short queries column groups and (token, query head) pairs.
     const int64_t entries = num_seqs * sq.vg;
     const int64_t columns = (int64_t)num_q_heads * sq.tpg;
-    RQ_CHECK_SPACE(workspace_bytes >= rq_fused_decode_workspace_bytes(entries, (int32_t)columns, head_dim, max_seq_len),
-                 "workspace too small");
+    const DecodeWorkspace W(entries, columns, sq.cu_q != nullptr ? num_kv_heads : num_q_heads, std::max<int64_t>(max_seq_len, 1));
+    RQ_CHECK_SPACE(workspace_bytes >= W.total, "workspace too small");
     RQ_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace % 16) == 0, "workspace must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
     DecodeArgs a{};
@@ -1556,7 +1558,6 @@ static int fused_decode_impl(const void *q, int32_t dtype, int64_t num_seqs, int
     a.rot_block = rot_block;
     a.score_scale = sm_scale * kLog2e;
     {
-        const DecodeWorkspace W(entries, columns, std::max<int64_t>(max_seq_len, 1));
         uint8_t *base = reinterpret_cast<uint8_t *>(workspace);
         a.part_acc = reinterpret_cast<float *>(base + W.part_acc);
         a.part_ml = reinterpret_cast<float *>(base + W.part_ml);
@@ -1688,7 +1689,7 @@ extern "C" int64_t rq_short_attention_workspace_bytes(int64_t num_seqs, int32_t 
     const ShortQueries sq = short_shape(num_q_heads, num_kv_heads, max_q_len);
     // (entries are a grid's y dimension in the merge, and divided as 32-bit numbers)
     if (sq.tpg == 0 || num_seqs < 0 || num_seqs * sq.vg > 65535) return 0;
-    return rq_fused_decode_workspace_bytes(num_seqs * sq.vg, num_q_heads * sq.tpg, kD, max_seq_len);
+    return DecodeWorkspace(num_seqs * sq.vg, (int64_t)num_q_heads * sq.tpg, num_kv_heads, std::max<int64_t>(max_seq_len, 1)).total;
 }
 
 extern "C" int rq_short_attention(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,

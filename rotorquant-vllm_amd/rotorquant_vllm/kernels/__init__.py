@@ -429,7 +429,8 @@ def _prefill_workspace(dev, workspace, need: int, split: int, short: int) -> tup
 
 # Workspace above which a call keeps the kernels that need none or less of it (the
 # partials take 0.5 KB per (token, head) column and workgroup, the descriptors 8.5
-# bytes per key of the bound on the lengths and column group).
+# bytes per key of the bound on the lengths and column group).  32 / 8 heads, 8 tokens each: reached by 128
+# sequences at a bound of 80000 keys, by 64 at 172000, by 32 at 356000.
 _SHORT_WORKSPACE_LIMIT = 256 << 20
 
 # Which kernels take a call of at most 16 tokens per sequence: the ones with the least estimated GPU time (us), as

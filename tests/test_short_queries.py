@@ -109,11 +109,31 @@ def test_short_queries_take_the_faster_kernels(launches, shape, attention, prefi
 
 @pytest.mark.parametrize("entry", ["paged_attention"] + PREFILLS)
 def test_calls_outside_the_short_kernels_keep_their_own(launches, entry):
-    """Longer queries, more groups of columns than the kernels take, scratch over the limit, no sequences."""
+    """Longer queries, more groups of columns than the kernels take, no sequences."""
     own = {"paged_attention": "rq_paged_attention", "fused_paged_rq_int8_prefill": "rq_int8_prefill", "paged_prefill": "rq_paged_prefill"}[entry]
-    for shape in ((4, 8, 32, 17, 4000), (4, 1, 9, 5, 4000), (4, 8, 64, 9, 4000), (128, 8, 32, 16, 1024), (0, 8, 32, 4, 4000)):
+    for shape in ((4, 8, 32, 17, 4000), (4, 1, 9, 5, 4000), (4, 8, 64, 9, 4000), (0, 8, 32, 4, 4000)):
         call(entry, *shape)
-    assert [x.name for x in launches] == [own] * 5
+    assert [x.name for x in launches] == [own] * 4
+
+
+@pytest.mark.parametrize("entry", ["paged_attention"] + PREFILLS)
+def test_scratch_of_short_calls_over_the_limit(launches, monkeypatch, entry):
+    """Calls that need more scratch than the limit keep kernels that need none or less."""
+    own = {"paged_attention": "rq_paged_attention", "fused_paged_rq_int8_prefill": "rq_int8_prefill", "paged_prefill": "rq_paged_prefill"}[entry]
+    need = _lib.load().rq_short_attention_workspace_bytes(4, 32, 8, 8, 4000)
+    for limit, name in ((need, "rq_short_attention"), (need - 1, own)):
+        monkeypatch.setattr(K, "_SHORT_WORKSPACE_LIMIT", limit)
+        call(entry, 4, 8, 32, 8, 4000)
+        assert launches[-1].name == name
+
+
+def test_scratch_of_short_calls_is_what_they_write():
+    """32 sequences of 8 tokens at 32 / 8 heads: 64 groups of 128 columns.  Query operands are 4 KB per group and kv head
+    (2 MB), beside the partials (520 bytes per column and slot, at most 4 slots per CU and one per group) and the
+    descriptors (272 bytes per 32 keys and group)."""
+    need = _lib.load().rq_short_attention_workspace_bytes(32, 32, 8, 8, 8000)
+    parts = [64 * 8 * 4096, (4 * 256 + 64) * 128 * 520, 64 * 250 * 272]
+    assert sum(parts) <= need <= sum(parts) + 16384
 
 
 @pytest.mark.parametrize("host_copies", [True, False])
