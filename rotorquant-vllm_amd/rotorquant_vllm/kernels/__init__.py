@@ -608,7 +608,7 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
                     v_centroids: torch.Tensor, rotation: torch.Tensor, num_kv_heads: int, head_dim: int,
                     block_size: int, sm_scale: float | None = None, causal: bool = True,
                     out: torch.Tensor | None = None, dense3: bool = False,
-                    max_seq_len: int | None = None) -> torch.Tensor:
+                    max_seq_len: int | None = None, workspace: torch.Tensor | None = None) -> torch.Tensor:
     """Attention of the new query tokens over the packed cache, q and output in original space.
 
     The reference's non-fused path (rq_backend.py:937-1036: q_rot = q R^T cast to
@@ -622,7 +622,10 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     index layout.  max_seq_len: a host int bounding every seq_lens entry (default: the
     block table's capacity), by which calls of at most 16 tokens per sequence
     choose between the two; a table much wider than the contexts is taken at its width
-    without it.
+    without it.  workspace: scratch of the latter (rq_short_attention_workspace_bytes bytes;
+    a smaller one keeps the former) instead of an allocation of the call from torch's
+    allocator, up to 256 MB; a graph captured without torch's graph classes needs it,
+    since nothing else keeps the scratch for its replays.
     """
     num_tokens, H_Q, D = q.shape
     assert D == head_dim
@@ -652,10 +655,10 @@ def paged_attention(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.
     capacity = bt.shape[1] * block_size
     short_len = capacity if max_seq_len is None else min(max_seq_len, capacity)
     route, sneed = _short_route(L, H_Q, num_kv_heads, sl.numel(), int(max_q_len), short_len, kv_cache, kc, vc, out, False)
-    if route == "short":
+    if route == "short" and (workspace is None or workspace.numel() >= sneed):
         # scratch of this call alone, from the stream's allocator: the call stays usable on several
         # streams at once, as the workspace-free kernel is
-        ws = torch.empty(sneed, dtype=torch.uint8, device=dev)
+        ws = torch.empty(sneed, dtype=torch.uint8, device=dev) if workspace is None else workspace
         rc = L.rq_short_attention(*head, short_len, *tail, ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
         _lib.check(rc, "rq_short_attention")
         return out

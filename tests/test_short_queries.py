@@ -127,6 +127,15 @@ def test_scratch_of_short_calls_over_the_limit(launches, monkeypatch, entry):
         assert launches[-1].name == name
 
 
+def test_scratch_of_short_calls_given_by_the_caller(launches):
+    """paged_attention on the caller's scratch: large enough it is what the kernels get, else the one launch runs."""
+    need = _lib.load().rq_short_attention_workspace_bytes(4, 32, 8, 8, 4000)
+    for given, name, scratch in ((need, "rq_short_attention", need), (need + 64, "rq_short_attention", need + 64),
+                                 (need - 1, "rq_paged_attention", None), (0, "rq_paged_attention", None)):
+        call("paged_attention", 4, 8, 32, 8, 4000, workspace=torch.empty(given, dtype=torch.uint8))
+        assert (launches[-1].name, launches[-1].scratch) == (name, scratch)
+
+
 def test_scratch_of_short_calls_is_what_they_write():
     """32 sequences of 8 tokens at 32 / 8 heads: 64 groups of 128 columns.  Query operands are 4 KB per group and kv head
     (2 MB), beside the partials (520 bytes per column and slot, at most 4 slots per CU and one per group) and the
