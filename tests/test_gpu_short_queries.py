@@ -6,8 +6,8 @@ import numpy as np
 import pytest
 import torch
 
-from rq_testlib import Params
-from test_gpu_attention import _dev, attn_case
+from rq_testlib import Params, build_cache_oracle, check_tolerance, kv_config0, paged_layout
+from test_gpu_attention import _dev, attn_case, ref
 
 pytestmark = pytest.mark.gpu
 
@@ -54,5 +54,82 @@ def test_weights_cancel_where_values_agree(fn, H, HQ, longest):
     cache[other, 0, v] = slot[v]
     got = run(fn, case, causal=False)
     assert np.isfinite(got).all() and np.abs(got[:longest]).max() > 0
-    # the rows of the one-key sequence are equal to one another per query head's kv head
     assert np.array_equal(got[:longest], got[longest:])
+
+
+def drafts(cfg, H, HQ, longest, p, BS=16, dtype=torch.bfloat16):
+    """Queries of 1 to `longest` tokens: contexts at the query's own length (the first token sees one key), around the edges
+    of the 32- and 64-key tiles, ending a token into a tile, and long; sequences without tokens or keys."""
+    q_lens = [longest, 1, 0, max(1, longest - 1), longest, min(2, longest), longest, 0]
+    ctx = [longest, 1, 40, 33, 64, 31 + min(2, longest), 1500, 0]
+    return attn_case(cfg, q_lens, ctx, H, HQ, p, BS=BS, dtype=dtype)
+
+
+def check(got, case, tag, causal=True):
+    exp = ref(case, causal)
+    err, excess, cs = check_tolerance(got, exp, str(case["q"].dtype).replace("torch.", ""), rot_block=case["p"].blk)
+    print(f"{tag}: max_abs={err:.3e} excess_over_bound={excess:.3e} cos={cs:.7f}", flush=True)
+    assert np.isfinite(got).all() and excess <= 0 and cs >= 0.999, (tag, err, excess, cs)
+
+
+# 8, 4, 2, 1 and a run-time number of kv heads per workgroup of the decode kernels, on up to 8 columns and on more
+HEADS = [(8, 8, 8), (4, 8, 4), (2, 4, 4), (1, 4, 2), (3, 6, 4), (8, 32, 4), (4, 28, 8), (2, 16, 2), (1, 8, 2), (3, 24, 2)]
+
+
+@pytest.mark.parametrize("H,HQ,longest", HEADS)
+def test_short_attention_heads_and_layouts(H, HQ, longest):
+    """Each form against the oracle, and on a dense 3-bit cache of the same tokens bit for bit."""
+    p = Params("iso", 3, 3)
+    case = drafts(130 + HQ, H, HQ, longest, p)
+    got = run("rq_short_attention", case)
+    check(got, case, f"short-{H}-{HQ}-{longest}")
+    ctx = case["lens"].tolist()
+    bt, NB, slots = paged_layout(ctx, 16, 130 + HQ)
+    k, v = kv_config0(sum(ctx), H, 128, 130 + HQ)
+    dense = build_cache_oracle(k, v, np.concatenate(slots), NB, 16, p, dense3=True)
+    assert np.array_equal(bt, case["bt"])
+    assert np.array_equal(run("rq_short_attention", dict(case, cache=dense), dense3=True), got)
+
+
+@pytest.mark.parametrize("BS", [1, 12, 32])
+@pytest.mark.parametrize("H,HQ,longest,bits,dtype,causal", [(2, 8, 5, (4, 3), torch.float16, True), (8, 16, 4, (3, 4), torch.bfloat16, False)])
+def test_short_attention_block_sizes(BS, H, HQ, longest, bits, dtype, causal):
+    case = drafts(140 + BS, H, HQ, longest, Params("planar", *bits), BS=BS, dtype=dtype)
+    check(run("rq_short_attention", case, causal), case, f"short-blocks-{BS}", causal)
+
+
+def test_short_attention_strided_rows():
+    """Query and output rows at other strides than their widths give the bits of plain ones, and nothing else is written."""
+    case = drafts(150, 4, 16, 6, Params("iso", 3, 3))
+    plain = run("rq_short_attention", case)
+    n, HQ = case["q"].shape[:2]
+    q = torch.full((n, HQ + 1, 136), float("nan"), dtype=torch.bfloat16, device="cuda")
+    out = torch.full((n, HQ, 132), 7.0, dtype=torch.bfloat16, device="cuda")
+    q[:, :HQ, :128] = case["q"].cuda()
+    got = run("rq_short_attention", case, q=q[:, :HQ, :128], out=out[..., :128])
+    assert np.array_equal(got, plain) and (out[..., 128:] == 7.0).all()
+
+
+@pytest.mark.parametrize("fn", ["rq_short_attention", "rq_paged_attention"])
+def test_more_tokens_than_keys(fn):
+    """The tokens before the first key see none and give zeros."""
+    case = attn_case(89, [5, 3], [2, 40], 2, 8, Params("iso", 3, 3))
+    got = run(fn, case)
+    assert (got[:3] == 0).all() and (got[3:] != 0).any(axis=(1, 2)).all()
+    case["q_lens"], case["cu"], case["q"] = [2, 3], np.asarray([0, 2, 5], np.int32), case["q"][3:]
+    check(got[3:], case, fn)
+
+
+@pytest.mark.parametrize("H,HQ,longest,bits,dtype,causal", [
+    (8, 32, 16, (3, 3), torch.bfloat16, True),
+    (8, 32, 1, (4, 4), torch.float16, True),
+    (4, 28, 16, (3, 4), torch.bfloat16, False),
+    (2, 24, 9, (4, 3), torch.float16, True),      # 12 heads: two workgroups per kv head, more groups than the decode kernels take
+    (1, 9, 16, (3, 3), torch.bfloat16, True),     # 9 heads: three
+    (1, 1, 16, (3, 3), torch.bfloat16, False),
+])
+def test_one_launch_over_many_tiles(H, HQ, longest, bits, dtype, causal):
+    """rq_paged_attention on queries of at most 16 tokens: both tile buffers, the running maximum and V exponent over up to 24
+    tiles, the split of wide groups, waves that only decode tiles."""
+    case = drafts(160 + HQ, H, HQ, longest, Params("iso", *bits), dtype=dtype)
+    check(run("rq_paged_attention", case, causal), case, f"one-launch-{HQ}-{longest}", causal)
