@@ -146,7 +146,7 @@ __device__ __forceinline__ void attn_work_item(int &qblk, int &h, int64_t &seq) 
 
 // Running state of one wave's 16 query positions (one per lane column).
 // acc = sum P' V' and lsum = sum P' 2^-e_v carry the same factor 2^-e_run, so
-// out = acc / l; m_run is in the score's base-2 units divided by sq.
+// out = acc / l; m_run is in the score's base-2 units.
 struct AttnState {
     f32x4 acc[8];
     f32x4 lsum;  // row 0 (lanes g = 0, element 0): the row sum of the weights
@@ -169,24 +169,23 @@ __device__ __forceinline__ u32x4 rowsum_operand(int e_v, int col) {
 }
 
 // Online softmax over one tile and O^T += V'^T P'^T.
-//   s: this lane's 16 scores (masked ones -INFINITY); the base-2 score proper is
-//      s * s_unit * sq (s_unit: per tile, sq: per position);
+//   s: this lane's 16 scores (masked ones -INFINITY), in base 2 once multiplied by scale;
 //   e_v: the tile's V exponent, V' = V 2^-e_v in fp16 (|V'| below max|centroid|);
 //   vt: the tile's V'^T rows; koff0 / koff1: this lane's pieces g and 4 + g of row
 //       col (vt_piece(col, g), vt_piece(col, 4 + g));
 //   ones: the tile's row-sum operand (rowsum_operand(e_v, col), col = lane % 16).
-__device__ __forceinline__ void softmax_pv(AttnState &st, const float (&s)[16], float s_unit, float sq, int e_v,
+__device__ __forceinline__ void softmax_pv(AttnState &st, const float (&s)[16], float scale, int e_v,
                                            const uint8_t *vt, int koff0, int koff1, const u32x4 ones) {
     float tmax = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
-    tmax = rows_max(tmax) * s_unit;
+    tmax = rows_max(tmax) * scale;
     // Lazy running max: rescale only when a position's max exceeds m_run by more
     // than 8 in log2 units, so p <= 2^8 in between (P' = p 2^(e_v - e_run) <= 2^8
     // stays in fp16); acc and lsum are relative to the same m_run either way.
-    if (__any((tmax - st.m_run) * sq > 8.f)) {
+    if (__any(tmax - st.m_run > 8.f)) {
         const float m_new = fmaxf(st.m_run, tmax);
-        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((st.m_run - m_new) * sq);
+        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(st.m_run - m_new);
 #pragma unroll
         for (int m = 0; m < 8; ++m)
 #pragma unroll
@@ -206,15 +205,14 @@ __device__ __forceinline__ void softmax_pv(AttnState &st, const float (&s)[16], 
         st.lsum *= f;
         st.e_run = e_v;
     }
-    const float bias = (st.m_run == -INFINITY ? 0.f : -st.m_run * sq) + (float)(e_v - st.e_run);
-    const float usq = s_unit * sq;
+    const float bias = (st.m_run == -INFINITY ? 0.f : -st.m_run) + (float)(e_v - st.e_run);
     // k-step t takes the scores of key blocks 2t and 2t + 1, in the lane's order.
     u32x4 pop[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         float p[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * t + e], usq, bias));
+        for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * t + e], scale, bias));
         pop[t] = u32x4{pack_f16(p[0], p[1]), pack_f16(p[2], p[3]), pack_f16(p[4], p[5]), pack_f16(p[6], p[7])};
     }
     st.lsum = mfma_f16(ones, pop[0], st.lsum);

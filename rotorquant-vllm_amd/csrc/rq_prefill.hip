@@ -60,7 +60,7 @@ struct PrefillArgs {
     int64_t stride_block, stride_token;
     int block_size, bs_shift;
     int64_t num_blocks;
-    int H, G, HQ;
+    int H, G;
     int dense3;         // dense 3-bit index layout of the cache
     const int32_t *bt;
     int64_t bt_ss, max_blocks;
@@ -631,7 +631,6 @@ int prefill_call(bool fused, int causal, const void *q, int32_t dtype, int64_t t
     a.num_blocks = num_blocks;
     a.H = num_kv_heads;
     a.G = num_q_heads / num_kv_heads;
-    a.HQ = num_q_heads;
     a.dense3 = index_layout == RQ_INDEX_DENSE3;
     a.bt = block_table;
     a.bt_ss = bt_stride_seq;
