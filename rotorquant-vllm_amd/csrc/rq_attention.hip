@@ -21,9 +21,9 @@
 // aligned mask with seqused_k); otherwise all seq_lens[b] keys.
 //
 // One workgroup per (query block, kv head, sequence); its waves are (query
-// head of the GQA group, position group).  WIDE (some query is longer than 16 tokens):
-// groups of 32 positions and rq_prefill.hip's tile steps (rq_attn_tile.h), so that both kernels
-// give the same bits; else groups of 16.  The
+// head of the GQA group, position group).  Groups of 16 positions, or WIDE (most calls with a query of
+// more than 16 tokens): of 32, with rq_prefill.hip's tile steps (rq_attn_tile.h), so that both kernels
+// give the same bits where that one runs unsplit.  The
 // workgroup decodes each 64-key tile of its (sequence, kv head) from the
 // packed slots into a double-buffered LDS tile (K rows in the q dtype, fp16
 // V'^T rows): while tile t is computed, tile t+1's packed bytes are copied
@@ -456,19 +456,36 @@ extern "C" int rq_paged_attention(const void *q, int32_t dtype, int64_t total_q,
     // (the smallest split into equal parts of at most kMaxWaves heads).  When every query is
     // short (one 16-position group), the workgroup has kMaxWaves waves anyway: the waves past
     // the GQA group's only decode tiles, which is most of a decode-shaped call's time.
-    // Longer queries take groups of 32 positions, as many as make kMinWaves waves (they share
-    // the tile decode).
     a.hsplit = 1;
     while (a.G % a.hsplit != 0 || a.G / a.hsplit > kMaxWaves) ++a.hsplit;
     const int gw = a.G / a.hsplit;
-    const bool wide = max_q_len > kPQ;
-    a.npg = wide ? (kMinWaves + gw - 1) / gw : 1;
+    // Longer queries.  Where workgroups of kMaxWaves waves in groups of 16 positions do not fill the CUs and the contexts may
+    // be long, a call takes one workgroup's chain of tiles, and these are the shortest (32 query / 4 kv heads, 17 tokens
+    // behind 2000 keys: 128 us, 144 in groups of 32; 8 / 8 heads 122 and 128).  Else groups of 32 positions:
+    // n4 of them make kMinWaves waves, two such workgroups to a CU; with the CUs not filled by these, kMaxWaves waves share the
+    // tile decode (8 / 8 heads, 32 tokens behind 300 keys: 39 us with four waves, 31 with eight); n8 of them make kMaxWaves
+    // waves that attend, half as many decodes of a tile, where they do not fill the CUs twice or queries are long enough
+    // for a workgroup's positions (32 / 8 heads, 32 x 33 tokens behind 2000 keys: 202 -> 149 us; one of 3000 tokens 263 ->
+    // 217; but 64 x 17 behind 300 42 -> 60).  The line at 1024 keys is where rq_paged_prefill splits such calls into key
+    // chunks: below it both give the same bits.
+    const int n4 = (kMinWaves + gw - 1) / gw, n8 = std::max(1, kMaxWaves / gw);
+    auto workgroups = [&](int positions) { return (max_q_len + positions - 1) / positions * a.H * a.hsplit * num_seqs; };
+    const int64_t cus = device_cus();
+    const bool longer = max_q_len > kPQ;
+    const bool wide = longer && (workgroups(kPQ * n8) > cus || max_blocks * block_size < 1024);
+    int nwaves = kMaxWaves;
+    a.npg = longer ? n8 : 1;
+    if (wide && workgroups(kPW * n4) <= cus) {
+        a.npg = n4;
+    } else if (wide && workgroups(kPW * n8) > cus && max_q_len < 8 * kPW * n4 && n4 != n8) {
+        a.npg = n4;
+        nwaves = gw * n4;
+    }
     a.qb = (wide ? kPW : kPQ) * a.npg;
     a.ncomp = gw * a.npg;
     a.out = out;
     a.o_st = out_stride_tok;
     a.o_sh = out_stride_head;
-    const int nwaves = wide ? a.ncomp : kMaxWaves;
     dim3 grid((unsigned)((max_q_len + a.qb - 1) / a.qb), (unsigned)(a.H * a.hsplit), (unsigned)num_seqs);
     const size_t lds = kLdsBytes;
     hipStream_t st = (hipStream_t)stream;

@@ -133,3 +133,20 @@ def test_one_launch_over_many_tiles(H, HQ, longest, bits, dtype, causal):
     tiles, the split of wide groups, waves that only decode tiles."""
     case = drafts(160 + HQ, H, HQ, longest, Params("iso", *bits), dtype=dtype)
     check(run("rq_paged_attention", case, causal), case, f"one-launch-{HQ}-{longest}", causal)
+
+
+@pytest.mark.parametrize("H,HQ,q_lens,ctx", [
+    (2, 16, [17, 40, 1], [1100, 64, 900]),         # groups of 16: 8 heads, one group a workgroup
+    (1, 3, [33, 97, 16], [1500, 97, 40]),          # 3 heads, two groups
+    (2, 2, [129, 20], [1024 + 129, 20]),           # 1 head, eight
+    (2, 12, [50, 17], [300, 17]),                  # groups of 32, two waves that only decode tiles
+    (1, 2, [65, 200], [365, 200]),                 # two groups, four such waves
+    (8, 32, [260, 30, 257, 200], [260, 90, 300, 200]),   # two groups of four heads
+    (8, 32, [17, 3] * 20, [40, 5] * 20),                 # one, four waves
+    (8, 8, [33] * 36, [64] * 36),                        # four groups of one head, four waves
+])
+@pytest.mark.parametrize("dtype,causal", [(torch.bfloat16, True), (torch.float16, False)])
+def test_one_launch_longer_queries(H, HQ, q_lens, ctx, dtype, causal):
+    """rq_paged_attention's workgroup shapes for queries of more than 16 tokens."""
+    case = attn_case(170 + HQ, q_lens, ctx, H, HQ, Params("iso", 3, 4), dtype=dtype)
+    check(run("rq_paged_attention", case, causal), case, f"one-launch-longer-{HQ}", causal)
