@@ -326,9 +326,9 @@ def decode_config1_tp8_slice(steps=20):
 def unfused_call(inp, q, cu, max_q, paged_attention=False):
     """The backend's non-fused path over a prepared cache, as it dispatches: single-token
     decodes -> one rq_fused_decode call (max_seq_len = the block table's capacity, as the
-    backend launches it); other queries of at most 16 tokens -> one rq_paged_attention
+    backend launches it); other queries of at most 16 tokens -> one paged_attention
     call; longer ones -> one rq_paged_prefill call (workspaces allocated here, outside the
-    timed calls).  paged_attention=True: rq_paged_attention for the decodes too.  Decode
+    timed calls).  paged_attention=True: paged_attention for the decodes too.  Decode
     calls rotate over the cache copies of `inp` (call i reads copy i % copies), so that
     the last-level cache does not serve a step from the one before."""
     import torch
@@ -369,7 +369,7 @@ def unfused_call(inp, q, cu, max_q, paged_attention=False):
 def time_unfused(cfg, steps=5):
     """The non-fused path (K/V rounded to bf16) on config 1's decode batch as the backend
     dispatches it (rq_fused_decode; bytes as the fused decode's roofline; also
-    rq_paged_attention on the same batch) or config 3's causal prefill (rq_paged_prefill;
+    paged_attention on the same batch, which runs it on the decode kernels' short-query form) or config 3's causal prefill (rq_paged_prefill;
     algorithmic bf16 flops = 2 x the causal Q K^T + P V multiply-adds)."""
     import torch
     if cfg == 1:

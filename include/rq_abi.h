@@ -277,9 +277,10 @@ int rq_fused_decode_noalloc(const void *q, int32_t dtype, int64_t num_seqs, int3
  * q / out: total_q x num_q_heads x head_dim, strides as for rq_fused_decode
  * (q rows and the rotation 16-byte aligned).  max_q_len bounds every q_len_b; max_seq_len bounds every seq_lens[b] (keys
  * past it are not read).  workspace: rq_int8_prefill_workspace_bytes() bytes,
- * 16-byte aligned, no initialisation needed (two launches: a pack kernel
- * decodes the cache's K/V into tile images there, the attention kernel
- * streams them).  Other arguments as for rq_fused_decode.
+ * 16-byte aligned, no initialisation needed (a pack kernel decodes the cache's K/V into
+ * tile images there, the attention kernel streams them; a call of few query blocks also
+ * merges partials of key chunks if the workspace holds them:
+ * rq_prefill_split_workspace_bytes).  Other arguments as for rq_fused_decode.
  */
 int rq_int8_prefill(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,
                     int64_t q_stride_tok, int64_t q_stride_head,
@@ -323,7 +324,8 @@ int64_t rq_int8_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads, 
  * (8-byte aligned rows); head_dim 128; num_q_heads / num_kv_heads <= 16;
  * 1..16 centroids per codebook; rot_block 2 or 4.  Other arguments as for
  * rq_int8_prefill.  Every launch size depends only on num_seqs, max_q_len and
- * num_kv_heads, so the call can be captured in a HIP graph.
+ * num_kv_heads, and the workgroup's shape also on the table's capacity, so the call can be
+ * captured in a HIP graph.
  */
 int rq_paged_attention(const void *q, int32_t dtype, int64_t total_q, int32_t num_q_heads,
                        int64_t q_stride_tok, int64_t q_stride_head,
@@ -340,8 +342,8 @@ int rq_paged_attention(const void *q, int32_t dtype, int64_t total_q, int32_t nu
                        void *stream);
 
 /*
- * The non-fused path of rq_paged_attention, same arithmetic, in two launches for
- * long queries: a pack kernel decodes every 64-key tile of every (sequence, kv
+ * The non-fused path of rq_paged_attention, same arithmetic, in two launches (three with
+ * key chunks) for long queries: a pack kernel decodes every 64-key tile of every (sequence, kv
  * head) once into a tile image in the workspace (K and V in the q dtype, the
  * values rq_decompress writes; V scaled exactly into fp16 by a power of two),
  * and the attention kernel streams the images (Q K^T on the q dtype's MFMA,
@@ -380,7 +382,9 @@ int64_t rq_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t num_kv_heads,
  * blocks over the whole GPU: the tile images, and fp32 partials of the key chunks that
  * several workgroups then take of one query block (at most 35 MB more; the same bytes as
  * rq_int8_prefill_workspace_bytes for calls that fill the GPU by themselves).  With a
- * workspace between the two sizes, the calls run unsplit.
+ * workspace between the two sizes, the calls run unsplit.  The order of a split call's sums
+ * follows the number of chunks, so a sequence's bits then depend on the other sequences of
+ * its call and on the workspace; unsplit, they do not.
  */
 int64_t rq_prefill_split_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                                          int64_t max_q_len, int64_t max_seq_len);
@@ -390,7 +394,8 @@ int64_t rq_prefill_split_workspace_bytes(int64_t num_seqs, int32_t num_q_heads, 
  * kernels of rq_fused_decode: the (token, query head) pairs of a kv head share its
  * stream of packed keys, up to 16 pairs at a time, so nothing is unpacked to memory
  * and the batch's keys are split over the whole GPU.  Arithmetic of the decode
- * kernels (K and V in the q dtype, exact products, fp32 sums).
+ * kernels (K and V in the q dtype, exact products, fp32 sums), except that a row is divided by
+ * the sum of its weights as rounded to fp16 for P V.
  *
  * Replaces the same reference code as rq_paged_attention (rq_backend.py:937-1036).
  * Arguments as for rq_paged_prefill, with rq_fused_decode's restrictions: 8 or 16

@@ -25,8 +25,8 @@
 //   with 11-bit operands on both sides: V' = V * 2^-e_tile in fp16, V the
 //   reference's centroid * norm rounded to the q dtype (:224), 2^e_tile above the
 //   64-key tile's largest v norm, and P' = p * 2^(e_tile - e_run) in fp16, e_run
-//   the largest e_tile so far (acc is rescaled when it grows); the row sum is taken in
-//   fp32 before P' is rounded.
+//   the largest e_tile so far (acc is rescaled when it grows); the row sum is the fp32
+//   sum of P', the rounded weights.
 //
 // Two kernels per call:
 //   * prefill_pack_kernel decodes every 64-key tile of every (sequence, kv head)
@@ -37,7 +37,7 @@
 //     four consecutive (position group, query head) units of a (sequence, kv head).
 //     It streams the tile images of its sequence and kv head into a double-buffered
 //     LDS area with direct global -> LDS copies (the copy of tile t+1 runs while tile
-//     t is computed), so the inner loop is MFMA and softmax only (wide_tile in
+//     t is computed), so the inner loop is MFMA and softmax only (the wide_* steps of
 //     rq_attn_tile.h, with the MFMA layouts).
 #include <algorithm>
 #include <type_traits>
@@ -253,7 +253,7 @@ __device__ __forceinline__ QueryBlock query_block(const PrefillArgs &a, int64_t 
 // each has its own barriers, so one computes while the other waits): 64 accumulator, 64 score
 // and 32 query registers a lane.  Steps on 8 x 4096 causal, 32 / 8 heads, whole call: 16-position
 // waves at four per SIMD 1326 us; 32-position waves, one phase after the other 1337;
-// interleaved (step, below) 1375; R read from LDS instead of memory 1190; rotations without a
+// interleaved (step, below; measured again in the final form there) 1375; R read from LDS instead of memory 1190; rotations without a
 // branch per dim and one rounding 1173.  Without the tile copies it takes 1082, without the tile
 // loop about 250 (copies of two tiles, rotations and stores).
 template <int DT>
@@ -388,9 +388,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
         float l = 0.f;
         // Tile t+1's scores run on the matrix cores under tile t's exponentials, and tile t's
         // P V under the search for tile t+1's maximum: an MFMA occupies its unit for 32 cycles
-        // and leaves the wave free to issue about 7 vector instructions (4 MFMAs and 28 FMAs
-        // of each of two waves on a SIMD: 130 ns interleaved, 164 one after the other, 110
-        // for the MFMAs alone).  The compiler neither interleaves them by itself nor reads
+        // and leaves the wave free to issue about 7 vector instructions.  Against the same step one phase
+        // after the other (equal bits): 8 x 4096 1190 -> 1180 us, one prompt of 700 28.0 -> 27.4, 3 chunks of 1500
+        // behind 5000 and 40 decodes 423 -> 417.  The compiler neither interleaves them by itself nor reads
         // operands far enough ahead of an LDS read's latency, so each slot below is
         // fenced: an operand read, an MFMA, and a sixteenth of the vector work.
         constexpr int kAhead = 5;  // operand reads in flight

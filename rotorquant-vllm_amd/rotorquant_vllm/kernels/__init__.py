@@ -436,7 +436,7 @@ _SHORT_WORKSPACE_LIMIT = 256 << 20
 # Which kernels take a call of at most 16 tokens per sequence: the ones with the least estimated GPU time (us), as
 # functions of the heads, the number of sequences and the bound on their lengths.  Fitted to captured calls on MI355X, iso 3-bit:
 # 4 / 16 / 64 / 128 sequences, 2 to 16 tokens, 64 to 1024 keys, 8 x 4, 1 x 4, 4 x 7, 8 x 1 and 2 x 8 (kv heads x
-# query heads of each); the route chosen there is within 10 % of the best one at 99 points in 100.  32 / 8 heads, 8 tokens:
+# query heads of each); the route chosen there is within 11 % of the best one at 99 points in 100.  32 / 8 heads, 8 tokens:
 #   sequences x keys       one launch   short   prefill kernels (us)
 #   4 x 64 / 256 / 1024    9 / 19 / 59   18 / 20 / 31   13 / 18 / 33
 #   64 x 64 / 256 / 1024   12 / 26 / 76   45 / 55 / 77   20 / 39 / 122
@@ -676,7 +676,9 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Te
     """paged_attention's arithmetic (the reference's non-fused path, rq_backend.py:937-1036)
     in two launches for long queries (rq_paged_prefill): every 64-key tile of every
     (sequence, kv head) is decoded once into a tile image (K and V in q's dtype),
-    then streamed by the attention kernel.
+    then streamed by the attention kernel; a third merges the key chunks of calls with few
+    query blocks.  Calls of at most 16 tokens per sequence run on the decode kernels or in
+    one launch where that is faster.
 
     Arguments as for paged_attention; max_seq_len bounds every seq_lens entry
     (default: the block table's capacity) and sizes the workspace, which may be

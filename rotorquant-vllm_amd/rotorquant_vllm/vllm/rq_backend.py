@@ -137,10 +137,10 @@ try:
 except (ImportError, OSError, RuntimeError) as exc:
     logger.info("RotorQuant HIP kernels unavailable: %s", exc)
 
-# Queries of at most this many tokens take the non-fused path's one-launch kernel
-# (rq_paged_attention: one query block per (sequence, kv head), each tile decoded
-# once anyway); longer ones take rq_paged_prefill, which decodes each tile once
-# for all query blocks instead of once per block.
+# Queries of at most this many tokens take the non-fused path's paged_attention
+# (rq_paged_attention, one query block per (sequence, kv head), or the decode kernels on
+# short queries: neither needs host lengths); longer ones take rq_paged_prefill, which
+# decodes each tile once for all query blocks instead of once per block.
 RQ_UNFUSED_SHORT_Q = 16
 
 # Shapes the fused kernels take (checked again by the C ABI): head_dim 128, a
@@ -735,10 +735,10 @@ class RQAttentionImpl(_ImplBase):
         exact Q K^T products, fp32 sums -- and a decode sees its whole context, causal
         or not; the batch's tiles are split over the whole GPU, and the launch is
         capturable in a HIP graph).  Other queries of at most RQ_UNFUSED_SHORT_Q tokens
-        take one rq_paged_attention launch (K/V tiles dequantized to the q dtype in
-        LDS; no workspace, no host read of the metadata, capturable).  A batch with
+        take paged_attention (one launch that dequantizes K/V tiles in LDS, or the decode
+        kernels on scratch from torch's allocator; no read of device metadata, capturable).  A batch with
         longer queries sends its leading single-token decodes (vLLM orders decodes
-        first) to the decode kernel, the following short ones to rq_paged_attention
+        first) to the decode kernel, the following short ones to paged_attention
         and the rest to rq_paged_prefill (same arithmetic; each 64-key tile decoded
         once into the prefill workspace, in groups that fit it).  Other shapes: the
         device path _forward_unfused_torch."""
