@@ -150,3 +150,26 @@ def test_one_launch_longer_queries(H, HQ, q_lens, ctx, dtype, causal):
     """rq_paged_attention's workgroup shapes for queries of more than 16 tokens."""
     case = attn_case(170 + HQ, q_lens, ctx, H, HQ, Params("iso", 3, 4), dtype=dtype)
     check(run("rq_paged_attention", case, causal), case, f"one-launch-longer-{HQ}", causal)
+
+
+@pytest.mark.parametrize("fused", [True, False], ids=["fused", "unfused"])
+@pytest.mark.parametrize("ctx,q_lens", [([2000, 3000, 700, 40], [1, 4, 8, 2]), ([60, 90, 8, 33], [1, 16, 8, 3])], ids=["long", "short"])
+def test_backend_drafts(monkeypatch, fused, ctx, q_lens):
+    """Drafts after a decode in one forward of the backend, over contexts that take the decode kernels and over short ones:
+    the cache bytes and every row, and the shared workspaces as they were reserved."""
+    import oracle as O
+    from rotorquant_vllm import kernels as K
+    from test_gpu_backend import _mixed_setup
+    impl, p, c = _mixed_setup(monkeypatch, 8, 32, "iso", 3, "fast", ctx, q_lens, 180, fused=fused)
+    cache = _dev(c["cache0"])
+    impl._init_cg_buffers(cache, torch.bfloat16)
+    retired = len(K._ws_retired)
+    out = torch.full(c["q"].shape, float("nan"), dtype=torch.bfloat16, device="cuda")
+    impl.forward(None, _dev(c["q"]), _dev(c["k_new"]), _dev(c["v_new"]), cache, c["md"], output=out)
+    torch.cuda.synchronize()
+    assert len(K._ws_retired) == retired and np.array_equal(cache.cpu().numpy(), c["full_cache"])
+    exp = O.unfused_attention(c["q"].float().numpy(), np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32), c["full_cache"], c["bt"],
+                              np.asarray(ctx, np.int32), 8, 128, p.kc.numpy(), p.vc.numpy(), p.R.numpy(), 128 ** -0.5, "bfloat16")
+    got = out.float().cpu().numpy()
+    err, excess, cs = check_tolerance(got, exp, "bfloat16", rot_block=p.blk)
+    assert np.isfinite(got).all() and excess <= 0 and cs >= 0.999, (err, excess, cs)
